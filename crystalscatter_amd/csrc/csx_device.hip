@@ -853,8 +853,10 @@ __device__ void coop_window_sum64(const DevSet& d, const Window& W, const PixArg
 }
 
 // Tier 3: the full reflection lists (lattice_ref64's terms).  A non-finite total takes the
-// serial reference loop, which stops at the first infinite partial sum.
-__device__ void coop_full_sum64(const DevSet& d, const PixArgs& me, bool want, double& inten, double& radint) {
+// serial reference loop, which stops at the first infinite partial sum; that depends on the
+// order of the terms, so there the mirror image's sum (inten2) is taken on its own.
+__device__ void coop_full_sum64(const DevSet& d, const PixArgs& me, bool want, bool mir, double& inten, double& inten2,
+                                double& radint) {
     unsigned long long m = __ballot(want);
     const int lane = threadIdx.x & 63;
     const csx_scalars& s = d.s;
@@ -881,10 +883,18 @@ __device__ void coop_full_sum64(const DevSet& d, const PixArgs& me, bool want, d
         rad = wave_sum(rad);
         if (lane == l) {
             inten = acc;
+            inten2 = acc;
             radint = rad;
         }
     }
-    if (want && !isfinite(inten)) lattice_ref64(d, me.qx, me.qy, me.qz, me.q, me.width, inten, radint);
+    if (want && !isfinite(inten)) {
+        for (int k = mir ? 1 : 0; k >= 0; --k) {
+            const double sg = k ? -1.0 : 1.0;
+            lattice_ref64(d, sg * me.qx, sg * me.qy, me.qz, me.q, me.width, inten, radint);
+            if (k) inten2 = inten;
+        }
+        if (!mir) inten2 = inten;
+    }
 }
 
 // Isotropic (radial) peak sum in FP32, only needed when iso != 0.
@@ -1145,19 +1155,10 @@ __device__ double cyl_gauss_quad(const DevSet& d, double qa, double qb, int oc) 
 // ---------------------------------------------------------------------------
 // Pixel value of each combination
 // ---------------------------------------------------------------------------
-// P3: the pixel (its exact q vector is computed here unless the caller has it); rv: its
-// radial-table entry (midpoint grid, sphere kinds) or null.
-// MODE kHot: *cold reports a pixel that needs an FP64 path, with its state in *cp; kFix:
-// finishes such a pixel from *cp.
-template <int KIND, int PREC, int MODE = kFull>
-__device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigned long long* stats = nullptr,
-                                              const Radial* rv = nullptr, bool* cold = nullptr,
-                                              ColdPix* cp = nullptr) {
+// Pixel value of the kinds without a lattice.
+template <int KIND>
+__device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, double qy, double q, const Radial* rv) {
     const csx_scalars& s = d.s;
-    // The mixed FCC path with a radial entry needs only |q| and the pixel indices.
-    if (!(rv && (KIND == K_FCC || KIND == K_ISO_LAT) && PREC == CSX_PREC_MIXED)) need_q(s, P3);
-    const double qx = P3.qx, qy = P3.qy, qz = P3.qz;
-    const double q = rv ? rv->q : sqrt(qx * qx + qy * qy + qz * qz) + 0.000000001;
     if constexpr (KIND == K_SPHERE) {
         const double pq = rv ? rv->pq : pq_sphere(d, q);
         return s.base + s.i0 * (pq + s.iso * pq) + s.ifluc / (1 + q * q * s.rfluc * s.rfluc);
@@ -1206,59 +1207,89 @@ __device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigne
         }
         const double pq = pql * pq_cyl_transverse(d, q);
         return s.base + s.i0 * (pq + s.iso) + s.ifluc / (1 + q * q * s.rfluc * s.rfluc);
+    }
+}
+
+// Value v[0] of the pixel P3 (its exact q vector is computed here unless the caller has it) and,
+// with `mir`, v[1] of its mirror image (-ihex, -i); rv: its radial-table entry (midpoint grid,
+// radial kinds) or null.  Only the lattice kinds in mixed precision take mirror images: in the
+// midpoint grid the peak sum at -q is the one at q (each Friedel pair swaps its two terms), and
+// so is every factor of |q|; the oriented cylinder's rod factor is evaluated at both.
+// MODE kHot: *cold reports a pixel that needs an FP64 path, with its state in *cp; kFix:
+// finishes such a pixel from *cp.
+template <int KIND, int PREC, int MODE = kFull>
+__device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* v, bool mir,
+                                             unsigned long long* stats = nullptr, const Radial* rv = nullptr,
+                                             bool* cold = nullptr, ColdPix* cp = nullptr) {
+    const csx_scalars& s = d.s;
+    // The mixed FCC path with a radial entry needs only |q| and the pixel indices.
+    if (!(rv && (KIND == K_FCC || KIND == K_ISO_LAT) && PREC == CSX_PREC_MIXED)) need_q(s, P3);
+    const double qx = P3.qx, qy = P3.qy, qz = P3.qz;
+    const double q = rv ? rv->q : sqrt(qx * qx + qy * qy + qz * qz) + 0.000000001;
+    if constexpr (!lattice_kind(KIND)) {
+        v[0] = pixel_no_lattice<KIND>(d, qx, qy, q, rv);
     } else {
-        double pq, fq;
-        if constexpr (KIND == K_FCC) {
-            if (rv) {
-                pq = rv->pq;
-                fq = rv->fq;
-            } else if constexpr (PREC == CSX_PREC_MIXED) {
-                pq = pq_sphere_fast(d, q);
-                fq = fq_sphere_fast(d, q);
+        // P(q) and <F>^2 at the pixel (k = 0) or its mirror image (k = 1)
+        auto factors = [&](int k, double& pq, double& fq) {
+            if constexpr (KIND == K_FCC) {
+                if (rv) {
+                    pq = rv->pq;
+                    fq = rv->fq;
+                } else if constexpr (PREC == CSX_PREC_MIXED) {
+                    pq = pq_sphere_fast(d, q);
+                    fq = fq_sphere_fast(d, q);
+                } else {
+                    pq = pq_sphere(d, q);
+                    fq = fq_sphere(d, q);
+                }
+            } else if constexpr (KIND == K_ISO_LAT) {
+                // calc_GENERIC, isotropic cylinders (Source/sc_gpu_generic.h:64-74: formpq and formfq
+                // of the cylinder at |q|) and homogeneous cubes (:295-302: formpq, and fq = pq)
+                if (rv) {
+                    pq = rv->pq;
+                    fq = rv->fq;
+                } else if (lattice_cube(s.combo_key)) {
+                    pq = pq_cube(d, q);
+                    fq = pq;
+                } else {
+                    pq = pq_cyl_long_iso(d, q) * pq_cyl_transverse(d, q);
+                    fq = fq_cyl_long_iso(d, q) * fq_cyl_radial(d, q);
+                }
             } else {
-                pq = pq_sphere(d, q);
-                fq = fq_sphere(d, q);
+                // the transverse P(q) and the radial factor of <F>^2 depend on |q| only: from the
+                // radial table when there is one (the same functions of the same |q|)
+                const double pt = rv ? rv->pq : pq_cyl_transverse(d, q);
+                const double fr = rv ? rv->fq : fq_cyl_radial(d, q);
+                const double x = k ? -qx : qx, y = k ? -qy : qy;
+                double pl, fl;
+                switch (s.orcase) {
+                case 0:
+                    cyl_long_both(d, q, sqrt(s.cosphi * x * x + s.sinphi * y * y + 0.000000001),
+                                  x * s.cosphi * s.sintheta, y * s.sinphi * s.sintheta, pl, fl);
+                    break;
+                case 1: cyl_long_both(d, q, fabs(x), x, 0, pl, fl); break;
+                case 2: cyl_long_both(d, q, fabs(y), 0, y, pl, fl); break;
+                default: cyl_long_both(d, q, q, x, y, pl, fl); break;
+                }
+                pq = pl * pt;
+                fq = fl * fr;
             }
-        } else if constexpr (KIND == K_ISO_LAT) {
-            // calc_GENERIC, isotropic cylinders (Source/sc_gpu_generic.h:64-74: formpq and formfq
-            // of the cylinder at |q|) and homogeneous cubes (:295-302: formpq, and fq = pq)
-            if (rv) {
-                pq = rv->pq;
-                fq = rv->fq;
-            } else if (lattice_cube(s.combo_key)) {
-                pq = pq_cube(d, q);
-                fq = pq;
-            } else {
-                pq = pq_cyl_long_iso(d, q) * pq_cyl_transverse(d, q);
-                fq = fq_cyl_long_iso(d, q) * fq_cyl_radial(d, q);
-            }
-        } else {
-            // the transverse P(q) and the radial factor of <F>^2 depend on |q| only: from the
-            // radial table when there is one (the same functions of the same |q|)
-            const double pt = rv ? rv->pq : pq_cyl_transverse(d, q);
-            const double fr = rv ? rv->fq : fq_cyl_radial(d, q);
-            double pl, fl;
-            switch (s.orcase) {
-            case 0:
-                cyl_long_both(d, q, sqrt(s.cosphi * qx * qx + s.sinphi * qy * qy + 0.000000001),
-                              qx * s.cosphi * s.sintheta, qy * s.sinphi * s.sintheta, pl, fl);
-                break;
-            case 1: cyl_long_both(d, q, fabs(qx), qx, 0, pl, fl); break;
-            case 2: cyl_long_both(d, q, fabs(qy), 0, qy, pl, fl); break;
-            default: cyl_long_both(d, q, q, qx, qy, pl, fl); break;
-            }
-            pq = pl * pt;
-            fq = fl * fr;
-        }
+        };
         double width = 1;
         if (s.dsch) width = 4.0 / s.domainsize;
         if (s.para) width = (4.0 / s.domainsize) + sqd(s.reldis) * s.dist * sqd(q);
         width *= s.width_zuf;
         double inten, radint;
         const double dwe = rv ? rv->dwe : exp(-s.dwfactor * q * q);
-        const double fqpq = fq / pq;
+        // the factors follow the peak sum, so that they do not occupy registers during it
+        constexpr int NV = KIND == K_BCT && PREC == CSX_PREC_MIXED ? 2 : 1;
+        double pq[NV], fqpq[NV], inten2;
         if constexpr (PREC == CSX_PREC_REF64) {
             lattice_ref64(d, qx, qy, qz, q, width, inten, radint);
+            inten2 = inten;
+            double fq;
+            factors(0, pq[0], fq);
+            fqpq[0] = fq / pq[0];
         } else {
             bool need_exact = false;
             double dropped = 0.0;
@@ -1286,6 +1317,17 @@ __device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigne
                             : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, stats);
             }
             radint = (s.iso != 0) ? iso_mixed(d, q) : 0.0;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                if (k == 0 || mir) {
+                    double fq;
+                    factors(k, pq[k], fq);
+                    fqpq[k] = fq / pq[k];
+                } else {
+                    pq[k] = pq[0];
+                    fqpq[k] = fqpq[0];
+                }
+            }
             // Conditioning guard.  szq = 1 + B - (fq/pq)*dwe with B = (fq/pq)*(2*pi*I/V)*dwe.
             // The peak sum I carries up to kRelErrFP32 (FP32 loop) or kRelErrPrecise (precise
             // loop) relative error plus this lane's dropped mass; szq amplifies an error of I
@@ -1293,12 +1335,17 @@ __device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigne
             // more than 3e-5 relative (and 2^-60 absolute, below the rounding of szq's own
             // FP64 terms) takes the same window in FP64, whose only error is the dropped mass;
             // if that is still too coarse, the reference's full FP64 sum, in its order.
-            const double bs = fqpq * d.two_pi_over_v * dwe;
             const double inv_hpw = s.para ? 1.0 / (kPiD * width / 2.0) : d.inv_hpw;
             auto loose = [&](double I, double rel) {
-                const double szq_est = 1 + fqpq * (I * d.two_pi_over_v - 1) * dwe;
-                const double dsz = fabs(bs) * (rel * fabs(I) + dropped * inv_hpw);
-                return !(dsz <= fmax(3.0e-5 * fabs(szq_est), 0x1p-60));
+                bool any = false;
+#pragma unroll
+                for (int k = 0; k < NV; ++k) {
+                    const double bs = fqpq[k] * d.two_pi_over_v * dwe;
+                    const double szq_est = 1 + fqpq[k] * (I * d.two_pi_over_v - 1) * dwe;
+                    const double dsz = fabs(bs) * (rel * fabs(I) + dropped * inv_hpw);
+                    any = any || !(dsz <= fmax(3.0e-5 * fabs(szq_est), 0x1p-60));
+                }
+                return any;
             };
             // placeholder lanes of the fix pass take no FP64 path
             const bool live = MODE != kFix || !(cp->flags & 4);
@@ -1306,32 +1353,44 @@ __device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigne
             if constexpr (MODE == kHot) {
                 *cold = W.near || need_exact || want2;
                 *cp = ColdPix{P3.ihex, P3.i, inten, dropped, W.b0, W.b1, W.band0, W.band1,
-                              (W.near ? 1 : 0) | (need_exact ? 2 : 0), 0};
+                              (W.near ? 1 : 0) | (need_exact ? 2 : 0) | (mir ? 8 : 0), 0};
+                inten2 = inten;
             } else {
-            if (__ballot(want2)) {
-                if (want2) need_q(s, P3);
-                coop_window_sum64<kPrecise>(d, W, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want2, inten);
-                if (stats && want2) atomicAdd(&stats[1], 1ull);
-            }
-            const bool want3 = need_exact || (want2 && loose(inten, 1.0e-13));
-            if (__ballot(want3)) {
-                if (want3) need_q(s, P3);
-                coop_full_sum64(d, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want3, inten, radint);
-                if (stats && want3) atomicAdd(&stats[4], 1ull);
-            }
+                if (__ballot(want2)) {
+                    if (want2) need_q(s, P3);
+                    coop_window_sum64<kPrecise>(d, W, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want2, inten);
+                    if (stats && want2) atomicAdd(&stats[1], 1ull);
+                }
+                const bool want3 = need_exact || (want2 && loose(inten, 1.0e-13));
+                inten2 = inten;
+                if (__ballot(want3)) {
+                    if (want3) need_q(s, P3);
+                    coop_full_sum64(d, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want3, mir, inten, inten2, radint);
+                    if (stats && want3) atomicAdd(&stats[4], 1ull);
+                }
             }
         }
-        const double szq = (1 + fqpq * (2 * kPiD * inten / s.sphno_cubevol - 1) * dwe);
-        const double pqiso = (KIND == K_FCC) ? pq : 1.0;
-        // iso == 0 and ifluc == 0 make their terms exactly +0 (szqiso is finite): skipped.
-        double isot = 0.0, fluct = 0.0;
-        if (s.iso != 0) {
-            const double szqiso = (1 + (1) * (8 * kPiD * kPiD * kPiD * radint / (4 * kPiD * s.sphno_cubevol) - 1) *
-                                           exp(-s.ucb * q * q));
-            isot = s.iso * szqiso * pqiso;
+        auto finish = [&](double pq1, double fqpq1, double I) {
+            const double szq = (1 + fqpq1 * (2 * kPiD * I / s.sphno_cubevol - 1) * dwe);
+            const double pqiso = (KIND == K_FCC) ? pq1 : 1.0;
+            // iso == 0 and ifluc == 0 make their terms exactly +0 (szqiso is finite): skipped.
+            double isot = 0.0, fluct = 0.0;
+            if (s.iso != 0) {
+                const double szqiso = (1 + (1) * (8 * kPiD * kPiD * kPiD * radint / (4 * kPiD * s.sphno_cubevol) - 1) *
+                                               exp(-s.ucb * q * q));
+                isot = s.iso * szqiso * pqiso;
+            }
+            if (s.ifluc != 0) fluct = s.ifluc / (1 + q * q * s.rfluc * s.rfluc);
+            return s.base + s.i0 * (szq * pq1 + isot) + fluct;
+        };
+        v[0] = finish(pq[0], fqpq[0], inten);
+        // the mirror image's value is the same unless a factor or a non-finite sum differs
+        v[1] = v[0];
+        if constexpr (PREC == CSX_PREC_MIXED) {
+            if (NV > 1 || MODE != kHot) {
+                if (mir && (NV > 1 || !isfinite(inten))) v[1] = finish(pq[NV - 1], fqpq[NV - 1], inten2);
+            }
         }
-        if (s.ifluc != 0) fluct = s.ifluc / (1 + q * q * s.rfluc * s.rfluc);
-        return s.base + s.i0 * (szq * pq + isot) + fluct;
     }
 }
 
@@ -1339,13 +1398,62 @@ __device__ __forceinline__ double pixel_value(const DevSet& d, PixQ& P3, unsigne
 // Kernels
 // ---------------------------------------------------------------------------
 
-// Image: tile (blockIdx.x, blockIdx.y) of the grid box; store in IDX order.
 // Pixel (px, py) of a 16x16 tile handled by lane threadIdx.x: each wave covers an 8x8
 // quadrant, the most compact 64-pixel footprint (narrowest |q| and angle ranges per wave).
 __device__ __forceinline__ void tile_pixel(int& px, int& py) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     px = (w & 1) * 8 + (l & 7);
     py = (w >> 1) * 8 + (l >> 3);
+}
+
+// How the workgroups of a launch cover a block of pixels, ihex in [x0, x1), i in [y0, y1).
+// Plain: one 16x16 tile each.  With mirror images (x0 = -x1, y0 = -y1): tiles over the rows
+// i < 0 only, each lane's value serving (ihex, i) and (-ihex, -i); the row i = 0 left of and
+// at the axis, and the column ihex = x0 below it (whose mirror images lie outside the block),
+// follow as workgroups of 256 consecutive pixels.  That is 2 z^2 + 2 z of 4 z^2 pixels.
+struct Cover {
+    int32_t x0, x1, y0, y1;
+    int32_t mirror, tiles_x, main, total;  // main: 16x16 tiles; total: workgroups
+};
+__host__ __device__ inline Cover make_cover(int x0, int x1, int y0, int y1, bool mirror) {
+    Cover c{x0, x1, y0, y1, mirror ? 1 : 0, 0, 0, 0};
+    c.tiles_x = (x1 - x0 + kTile - 1) / kTile;
+    c.main = c.tiles_x * (((mirror ? -y0 : y1 - y0) + kTile - 1) / kTile);
+    c.total = c.main + (mirror ? (x1 + y1 + kBlock - 1) / kBlock : 0);
+    return c;
+}
+struct CoverPix {
+    int ihex, i;
+    bool in, mir;  // the lane has a pixel of the block; its mirror image is this lane's as well
+};
+// Lanes without a pixel repeat a neighbouring one (the mixed path needs all 64 lanes).
+__device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t) {
+    CoverPix p;
+    if (t < c.main) {
+        int px, py;
+        tile_pixel(px, py);
+        const int ylim = c.mirror ? 0 : c.y1;
+        const int ihex = c.x0 + t % c.tiles_x * kTile + px, i = c.y0 + t / c.tiles_x * kTile + py;
+        p.in = ihex < c.x1 && i < ylim;
+        p.ihex = min(ihex, c.x1 - 1);
+        p.i = min(i, ylim - 1);
+        p.mir = c.mirror && p.in && ihex > c.x0 && i > c.y0;
+    } else {
+        const int n = (t - c.main) * kBlock + (int)threadIdx.x;
+        p.in = n < c.x1 + c.y1;
+        const int k = min(n, c.x1 + c.y1 - 1);
+        const bool row = k <= c.x1;
+        p.ihex = row ? c.x0 + k : c.x0;
+        p.i = row ? 0 : k - c.x1;
+        p.mir = p.in && row && k > 0 && k < c.x1;
+    }
+    return p;
+}
+// Mirror images serve the lattice kinds' Gaussian peak sums in mixed precision, in the
+// midpoint grid, when every reflection has its Friedel partner in the list.
+inline bool mirror_set(const DevSet& d, int kind, int precision, int x0, int x1, int y0, int y1) {
+    return lattice_kind(kind) && precision == CSX_PREC_MIXED && d.nsingle == 0 && !d.s.centerbeam && !d.s.use1d &&
+           x1 > 0 && y1 > 0 && x0 == -x1 && y0 == -y1;
 }
 
 // Kinds whose form factors depend on |q| only.
@@ -1416,37 +1524,35 @@ __global__ void __launch_bounds__(256) k_radial(const DevSet d, int m, Radial* _
     radial_block<KIND, PREC>(d, m, tab, blockIdx.x);
 }
 
-// Image: tile (blockIdx.x, blockIdx.y) of the grid box; store in IDX order.  rtab: radial
-// table of k_radial (midpoint grid, radial kinds) or null.
+// Image: workgroup `t` of the cover; store in IDX order.  rtab: radial table of k_radial
+// (midpoint grid, radial kinds) or null.
 template <int KIND, int PREC, int MODE = kFull>
-__device__ __forceinline__ void image_tile(const DevSet& d, const csx_grid& g, double* __restrict__ out,
+__device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, double* __restrict__ out,
                                            unsigned long long* __restrict__ stats, const Radial* __restrict__ rtab,
                                            ColdQueue cq = ColdQueue{}) {
-    // Every lane computes (the mixed path needs all 64 lanes of a wave); lanes past the grid
-    // edge evaluate the last valid pixel, and only in-grid pixels are stored.
-    int px, py;
-    tile_pixel(px, py);
-    const int ihex0 = g.xmin + blockIdx.x * kTile + px;
-    const int i0 = g.ymin + blockIdx.y * kTile + py;
-    const int ihex = min(ihex0, g.xmax - 1), i = min(i0, g.ymax - 1);
-    PixQ P3{ihex, i, 0.0, 0.0, 0.0, false};
+    const int t = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    if (t >= c.total) return;
+    const CoverPix p = cover_pixel(c, t);
+    PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
     if constexpr (KIND == K_CYL_GAUSS_Q) {
         for (int k = threadIdx.x; k <= kCqTab; k += kBlock) g_cq_tab[k] = d.cq_tab[k];
         if (threadIdx.x < kCqDelta) g_cq_dl[threadIdx.x] = d.cq_delta[threadIdx.x];
         if (threadIdx.x < kCqPsi / 2) g_cq_tt[threadIdx.x] = d.cq_t[threadIdx.x];
         __syncthreads();
     }
+    if (!__ballot(p.in)) return;
     const Radial* rv = nullptr;
     if (rtab) {
-        const int a = abs(i), b = abs(ihex);
+        const int a = abs(p.i), b = abs(p.ihex);
         rv = rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
     }
     bool cold = false;
     ColdPix cpx;
-    const double v = pixel_value<KIND, PREC, MODE>(d, P3, stats, rv, &cold, &cpx);
+    double v[2];
+    pixel_values<KIND, PREC, MODE>(d, P3, v, p.mir, stats, rv, &cold, &cpx);
     if constexpr (MODE == kHot) {
-        // queue the in-grid cold pixels (lanes past the edge repeat an in-grid pixel)
-        const bool mine = cold && ihex0 < g.xmax && i0 < g.ymax;
+        // queue the cold pixels (lanes without a pixel repeat one)
+        const bool mine = cold && p.in;
         const unsigned long long m = __ballot(mine);
         if (m) {
             const int lane = threadIdx.x & 63;
@@ -1459,24 +1565,17 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const csx_grid& g, d
             if (mine) cq.ent[(size_t)slot * 64 + lane] = cpx;
         }
     }
-    // Stage the tile in LDS and store it row by row: each wave then writes four whole rows of
-    // 16 doubles (full 128-byte lines) instead of half lines from its 8x8 quadrant.
-    __shared__ double tile[kTile][kTile + 1];
-    tile[py][px] = v;
-    __syncthreads();
-    const int r = threadIdx.x / kTile, cx = threadIdx.x % kTile;
-    const int oh = g.xmin + blockIdx.x * kTile + cx, oi = g.ymin + blockIdx.y * kTile + r;
-    if (oh < g.xmax && oi < g.ymax) {
-        const size_t W = (size_t)(g.xmax - g.xmin);
-        out[(size_t)(oh - g.xmin) + W * (size_t)(oi - g.ymin)] = tile[r][cx];
-    }
+    // 64-byte row segments; the other half of each line is written by the same workgroup
+    const size_t W = (size_t)(c.x1 - c.x0);
+    if (p.in) out[(size_t)(p.ihex - c.x0) + W * (size_t)(p.i - c.y0)] = v[0];
+    if (p.mir) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[1];
 }
 
 template <int KIND, int PREC>
-__global__ void __launch_bounds__(kBlock) k_image(const DevSet d, const csx_grid g, double* __restrict__ out,
+__global__ void __launch_bounds__(kBlock) k_image(const DevSet d, const Cover c, double* __restrict__ out,
                                                   unsigned long long* __restrict__ stats,
                                                   const Radial* __restrict__ rtab) {
-    image_tile<KIND, PREC>(d, g, out, stats, rtab);
+    image_tile<KIND, PREC>(d, c, out, stats, rtab);
 }
 
 // Lattice kinds in one pass (sets with unpaired reflections, where every pixel takes an FP64
@@ -1485,9 +1584,9 @@ __global__ void __launch_bounds__(kBlock) k_image(const DevSet d, const csx_grid
 // SIMD), only those cold paths spill.
 template <int KIND, int PREC>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
-k_image_lat(const DevSet d, const csx_grid g, double* __restrict__ out, unsigned long long* __restrict__ stats,
+k_image_lat(const DevSet d, const Cover c, double* __restrict__ out, unsigned long long* __restrict__ stats,
             const Radial* __restrict__ rtab) {
-    image_tile<KIND, PREC>(d, g, out, stats, rtab);
+    image_tile<KIND, PREC>(d, c, out, stats, rtab);
 }
 
 // Lattice kinds, two passes.  The hot pass carries no FP64 re-sum code (no spills, more waves
@@ -1495,18 +1594,18 @@ k_image_lat(const DevSet d, const csx_grid g, double* __restrict__ out, unsigned
 // with the same arithmetic as the one-pass kernel, so every pixel is bitwise the same.
 template <int KIND, int PREC>
 __global__ void __launch_bounds__(kBlock)
-k_image_lat_hot(const DevSet d, const csx_grid g, double* __restrict__ out, unsigned long long* __restrict__ stats,
+k_image_lat_hot(const DevSet d, const Cover c, double* __restrict__ out, unsigned long long* __restrict__ stats,
                 const Radial* __restrict__ rtab, ColdQueue cq) {
-    image_tile<KIND, PREC, kHot>(d, g, out, stats, rtab, cq);
+    image_tile<KIND, PREC, kHot>(d, c, out, stats, rtab, cq);
 }
 
 template <int KIND, int PREC>
 __global__ void __launch_bounds__(64)
-k_image_lat_fix(const DevSet d, const csx_grid g, double* __restrict__ out, unsigned long long* __restrict__ stats,
+k_image_lat_fix(const DevSet d, const Cover c, double* __restrict__ out, unsigned long long* __restrict__ stats,
                 const Radial* __restrict__ rtab, ColdQueue cq) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *cq.next_count = 0;
     const int n = *cq.count;
-    const size_t W = (size_t)(g.xmax - g.xmin);
+    const size_t W = (size_t)(c.x1 - c.x0);
     // one wave per slot (the FP64 re-sums are wave-cooperative); lanes without a cold pixel
     // repeat the slot's first one as placeholders
     for (int slot = blockIdx.x; slot < n; slot += gridDim.x) {
@@ -1514,6 +1613,7 @@ k_image_lat_fix(const DevSet d, const csx_grid g, double* __restrict__ out, unsi
         const int lane = (int)threadIdx.x;
         const bool have = (m >> lane) & 1ull;
         ColdPix cp = cq.ent[(size_t)slot * 64 + (have ? lane : __builtin_ctzll(m))];
+        const bool mir = have && (cp.flags & 8);
         if (!have) cp.flags = 4;
         PixQ P3{cp.ihex, cp.i, 0.0, 0.0, 0.0, false};
         const Radial* rv = nullptr;
@@ -1521,8 +1621,10 @@ k_image_lat_fix(const DevSet d, const csx_grid g, double* __restrict__ out, unsi
             const int a = abs(cp.i), b = abs(cp.ihex);
             rv = rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
         }
-        const double v = pixel_value<KIND, PREC, kFix>(d, P3, stats, rv, nullptr, &cp);
-        if (have) out[(size_t)(cp.ihex - g.xmin) + W * (size_t)(cp.i - g.ymin)] = v;
+        double v[2];
+        pixel_values<KIND, PREC, kFix>(d, P3, v, mir, stats, rv, nullptr, &cp);
+        if (have) out[(size_t)(cp.ihex - c.x0) + W * (size_t)(cp.i - c.y0)] = v[0];
+        if (mir) out[(size_t)(-cp.ihex - c.x0) + W * (size_t)(-cp.i - c.y0)] = v[1];
     }
 }
 
@@ -1581,7 +1683,8 @@ struct FitSet {
     csx_mask m;
     const double* data;
     int32_t w, h;
-    int32_t tiles_x, first_tile;  // tile range of this set in the batch
+    Cover cov;                    // the fit array's pixels, from (iimin, iimin)
+    int32_t first_tile, pad_tile; // the set's first workgroup in the batch
     const Radial* rtab;           // radial table of the set (k_batch_radial), or null
     int32_t rad_m, rad_pad;       // its largest |index|
     PrepIn pin;
@@ -1598,55 +1701,51 @@ struct TileSum {
 // sets array, the isotropic cylinder's P(q) came out wrong above its series radius (with and
 // without a lattice).  The sphere and z-oriented cylinder lattice kinds read them in place.
 template <int KIND, int PREC>
-__device__ __forceinline__ double set_pixel(const FitSet& f, PixQ& P3, const Radial* rv) {
+__device__ __forceinline__ void set_pixel(const FitSet& f, PixQ& P3, double* v, bool mir, const Radial* rv) {
     if constexpr (KIND == K_FCC || KIND == K_BCT) {
-        return pixel_value<KIND, PREC>(f.d, P3, nullptr, rv);
+        pixel_values<KIND, PREC>(f.d, P3, v, mir, nullptr, rv);
     } else {
         const DevSet d = f.d;
-        return pixel_value<KIND, PREC>(d, P3, nullptr, rv);
+        pixel_values<KIND, PREC>(d, P3, v, mir, nullptr, rv);
     }
 }
 
-// One fit tile: per-pixel FQSVERGL terms, NaN counted, block-reduced in FP64.
+// One workgroup of a set's cover: per-pixel FQSVERGL terms, NaN counted, block-reduced in FP64.
 template <int KIND, int PREC>
 __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __restrict__ fqs_out, TileSum* __restrict__ out) {
     __shared__ double s_sum[kBlock / 64];
     __shared__ int s_cnt[kBlock / 64], s_nan[kBlock / 64];
-    const int tx = tile % f.tiles_x, ty = tile / f.tiles_x;
-    int px, py;
-    tile_pixel(px, py);
-    const int x = tx * kTile + px;
-    const int y = ty * kTile + py;
     double term = 0.0;
     int nz = 0, isnan_ = 0;
-    // All lanes evaluate a pixel (wave-wide |q| ranges need all 64 lanes); lanes outside the
-    // fit array or masked discard the value.
-    const bool inside = x < f.w && y < f.h;
-    const int xc = min(x, f.w - 1), yc = min(y, f.h - 1);
-    const csx_scalars& s = f.d.s;
-    const bool masked = !inside || fit_masked(s, f.m, f.data, f.w, xc, yc);
-    const int ihex = xc + s.iimin, i = yc + s.iimin;
-    PixQ P3{ihex, i, 0.0, 0.0, 0.0, false};
-    const Radial* rv = nullptr;
-    if (f.rtab) {
-        const int a = abs(i), b = abs(ihex);
-        rv = f.rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
-    }
-    const double v = set_pixel<KIND, PREC>(f, P3, rv);
-    if (inside) {
-        const size_t idx = (size_t)(ihex - s.xmin) + (size_t)(s.xmax - s.xmin) * (size_t)(i - s.ymin);
-        if (!masked) {
-            const double dv = f.data[idx];
-            if (v > 0 && dv > 0) {
-                const double a = log(v) / log(10.) - log(dv) / log(10.);
-                term = a * a;
-            }
-            if (fqs_out) fqs_out[idx] = term;
-        } else if (fqs_out) {
-            fqs_out[(size_t)x + (size_t)f.w * y] = 0.0;
+    const CoverPix p = cover_pixel(f.cov, tile);
+    // All lanes of a wave with a pixel evaluate one (wave-wide |q| ranges need all 64 lanes);
+    // lanes outside the fit array or masked discard the value.
+    if (__ballot(p.in)) {
+        const csx_scalars& s = f.d.s;
+        PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
+        const Radial* rv = nullptr;
+        if (f.rtab) {
+            const int a = abs(p.i), b = abs(p.ihex);
+            rv = f.rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
         }
-        if (isnan(term)) { isnan_ = 1; term = 0.0; }
-        else if (term != 0) nz = 1;
+        double v[2];
+        set_pixel<KIND, PREC>(f, P3, v, p.mir, rv);
+        for (int k = 0; k < 2; ++k) {
+            if (!(k ? p.mir : p.in)) continue;
+            const int x = (k ? -p.ihex : p.ihex) - f.cov.x0, y = (k ? -p.i : p.i) - f.cov.y0;
+            const size_t idx = (size_t)x + (size_t)f.w * (size_t)y;
+            double tk = 0.0;
+            if (!fit_masked(s, f.m, f.data, f.w, x, y)) {
+                const double dv = f.data[idx];
+                if (v[k] > 0 && dv > 0) {
+                    const double a = log(v[k]) / log(10.) - log(dv) / log(10.);
+                    tk = a * a;
+                }
+            }
+            if (fqs_out) fqs_out[idx] = tk;
+            if (isnan(tk)) ++isnan_;
+            else if (tk != 0) { ++nz; term += tk; }
+        }
     }
     const double ws = wave_sum(term);
     const int wc = wave_sum_i(nz), wn = wave_sum_i(isnan_);
@@ -1712,8 +1811,7 @@ k_fit_batch_cap(const FitSet* __restrict__ sets, const int2* __restrict__ tiles,
 }
 
 // Batched images: one launch over the flat tile list of many parameter sets, each set's
-// image (its whole grid, IDX order) written to the buffer staged as its data pointer.  The
-// tile goes through LDS so that every wave stores whole 128-byte rows.
+// image (its whole grid, IDX order) written to the buffer staged as its data pointer.
 template <int KIND, int PREC>
 __device__ __forceinline__ void image_batch_tiles(const FitSet* __restrict__ sets, const int2* __restrict__ tiles,
                                                   int ntiles) {
@@ -1721,24 +1819,19 @@ __device__ __forceinline__ void image_batch_tiles(const FitSet* __restrict__ set
     if (t >= ntiles) return;
     const int2 st = tiles[t];
     const FitSet& f = sets[st.x];
-    const int tx = st.y % f.tiles_x, ty = st.y / f.tiles_x;
-    int px, py;
-    tile_pixel(px, py);
-    const csx_scalars& s = f.d.s;
-    const int x = min(tx * kTile + px, f.w - 1), y = min(ty * kTile + py, f.h - 1);
-    PixQ P3{s.xmin + x, s.ymin + y, 0.0, 0.0, 0.0, false};
+    const CoverPix p = cover_pixel(f.cov, st.y);
+    if (!__ballot(p.in)) return;
+    PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
     const Radial* rv = nullptr;
     if (f.rtab) {
         const int a = abs(P3.i), b = abs(P3.ihex);
         rv = f.rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
     }
-    const double v = set_pixel<KIND, PREC>(f, P3, rv);
-    __shared__ double tile[kTile][kTile + 1];
-    tile[py][px] = v;
-    __syncthreads();
-    const int r = threadIdx.x / kTile, cx = threadIdx.x % kTile;
-    const int ox = tx * kTile + cx, oy = ty * kTile + r;
-    if (ox < f.w && oy < f.h) const_cast<double*>(f.data)[(size_t)ox + (size_t)f.w * oy] = tile[r][cx];
+    double v[2];
+    set_pixel<KIND, PREC>(f, P3, v, p.mir, rv);
+    double* out = const_cast<double*>(f.data);
+    if (p.in) out[(size_t)(p.ihex - f.cov.x0) + (size_t)f.w * (size_t)(p.i - f.cov.y0)] = v[0];
+    if (p.mir) out[(size_t)(-p.ihex - f.cov.x0) + (size_t)f.w * (size_t)(-p.i - f.cov.y0)] = v[1];
 }
 template <int KIND, int PREC>
 __global__ void __launch_bounds__(kBlock) k_image_batch(const FitSet* __restrict__ sets, const int2* __restrict__ tiles,
@@ -2570,8 +2663,8 @@ struct csx_ctx {
     long long pass_n = 0;                        // renders recorded into the ring
     // batch staging
     std::vector<FitSet> bsets;
-    std::vector<int> bntiles;
-    int bntiles_total = 0;  // tiles of the pending batch (its flat tile list is built on the device)
+    std::vector<int> bntiles;  // workgroups of each set in the batch's last launch
+    int bntiles_total = 0;     // 16x16 tiles of the pending batch's fit arrays (tuning size class)
     DevBuf btiles_d;
     PinnedArena barena;  // host image of the device arena (tables of all sets), pinned
     PinnedArena bres;    // sums and counts of the batch in flight (size = its set count)
@@ -2712,9 +2805,9 @@ constexpr int kFixBlocks = 256;
 
 // ev: null, or two events recorded around the per-pixel kernel (the hot pass when two).
 template <int K, int P>
-static void launch_image(const DevSet& d, const csx_grid& g, double* out, unsigned long long* stats,
+static void launch_image(const DevSet& d, const Cover& g, double* out, unsigned long long* stats,
                          const Radial* rtab, const ColdQueue* cq, hipEvent_t* ev, hipStream_t st) {
-    dim3 grid((g.xmax - g.xmin + kTile - 1) / kTile, (g.ymax - g.ymin + kTile - 1) / kTile);
+    const dim3 grid(g.tiles_x, (g.total + g.tiles_x - 1) / g.tiles_x);
     if (ev) (void)hipEventRecord(ev[0], st);
     if constexpr (lattice_kind(K) && P == CSX_PREC_MIXED) {
         if (cq) {
@@ -2743,6 +2836,11 @@ int csx_qgrid(csx_ctx* c, const csx_grid* g, double* d_q3) {
     return CSX_OK;
 }
 
+// Cover of a set's fit array.
+static Cover fit_cover(const FitSet& f, int kind, int precision) {
+    const int x0 = f.d.s.iimin;
+    return make_cover(x0, x0 + f.w, x0, x0 + f.h, mirror_set(f.d, kind, precision, x0, x0 + f.w, x0, x0 + f.h));
+}
 template <int K, int P>
 static void launch_fit_one(const FitSet& f, int ntiles, double* fqs, TileSum* part, hipStream_t st) {
     hipLaunchKernelGGL((k_fit_one<K, P>), dim3(ntiles), dim3(kBlock), 0, st, f, fqs, part);
@@ -2872,13 +2970,14 @@ static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g,
         HIPCHK(c, hipEventRecord(c->ev_rad[sl], c->side));
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_rad[sl], 0));
     }
+    const Cover cov = make_cover(g.xmin, g.xmax, g.ymin, g.ymax,
+                                 mirror_set(c->set, kind, precision, g.xmin, g.xmax, g.ymin, g.ymax));
     // Lattice kinds in mixed precision render in two passes (hot, then fix over a queue of at
     // most one slot per wave), unless unpaired reflections send every pixel to FP64.
     ColdQueue cq{};
     const ColdQueue* cqp = nullptr;
     if (lattice_kind(kind) && precision == CSX_PREC_MIXED && c->set.nsingle == 0) {
-        const size_t nwaves = 4 * (size_t)((g.xmax - g.xmin + kTile - 1) / kTile) *
-                              (size_t)((g.ymax - g.ymin + kTile - 1) / kTile);
+        const size_t nwaves = 4 * (size_t)cov.total;
         const size_t need = 256 + nwaves * (sizeof(unsigned long long) + 64 * sizeof(ColdPix));
         if (need > c->coldq.n) {
             HIPCHK(c, c->coldq.ensure(need));
@@ -2900,7 +2999,7 @@ static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g,
         ev = e;
         ++c->pass_n;
     }
-    DISPATCH_KIND(kind, precision, launch_image, c->set, g, out, stats, rtab, cqp, ev, c->stream);
+    DISPATCH_KIND(kind, precision, launch_image, c->set, cov, out, stats, rtab, cqp, ev, c->stream);
     HIPCHK(c, hipGetLastError());
     if (rtab) {
         HIPCHK(c, hipEventRecord(c->ev_img[sl], c->stream));
@@ -3198,12 +3297,12 @@ int csx_fit_fqs(csx_ctx* c, int w, int h, const csx_mask* mask, int precision_in
     f.data = d_data;
     f.w = w;
     f.h = h;
-    f.tiles_x = (w + kTile - 1) / kTile;
-    const int ntiles = f.tiles_x * ((h + kTile - 1) / kTile);
+    const int kind = kind_of(s.combo_key);
+    f.cov = fit_cover(f, kind, precision);
+    const int ntiles = f.cov.total;
     HIPCHK(c, c->tiles.ensure((size_t)ntiles * sizeof(TileSum) + sizeof(SetSum)));
     TileSum* part = (TileSum*)c->tiles.p;
     SetSum* total = (SetSum*)(part + ntiles);
-    const int kind = kind_of(s.combo_key);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     DISPATCH_KIND(kind, precision, launch_fit_one, f, ntiles, d_fqs, part, c->stream);
     HIPCHK(c, hipGetLastError());
@@ -3250,13 +3349,14 @@ int csx_fit_fqs_noalloc(csx_ctx* c, int w, int h, const csx_mask* mask, int prec
     f.data = d_data;
     f.w = w;
     f.h = h;
-    f.tiles_x = tiles_x;
     const int kind = kind_of(s.combo_key);
+    f.cov = fit_cover(f, kind, precision);  // never more workgroups than the checked tiles
+    if (f.cov.total > kScratchTiles) return fail(c, CSX_E_ARG, "csx_fit_fqs_noalloc: too many tiles");
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    DISPATCH_KIND(kind, precision, launch_fit_one, f, (int)ntiles, d_fqs, part, c->stream);
+    DISPATCH_KIND(kind, precision, launch_fit_one, f, f.cov.total, d_fqs, part, c->stream);
     HIPCHK(c, hipGetLastError());
     SetSum* d_total = (SetSum*)(part + kScratchTiles);
-    hipLaunchKernelGGL(k_sum_tiles, dim3(1), dim3(kBlock), 0, c->stream, part, (int)ntiles, d_total);
+    hipLaunchKernelGGL(k_sum_tiles, dim3(1), dim3(kBlock), 0, c->stream, part, f.cov.total, d_total);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     SetSum total{};
@@ -3352,8 +3452,7 @@ static bool stage_begin(csx_staged& st, const csx_scalars* s, const double* h_ca
     f.data = d_data;
     f.w = w;
     f.h = h;
-    f.tiles_x = (w + kTile - 1) / kTile;
-    st.ntiles = f.tiles_x * ((h + kTile - 1) / kTile);
+    st.ntiles = ((w + kTile - 1) / kTile) * ((h + kTile - 1) / kTile);
     auto& pd = st.pd;
     pd = csx_staged::Offsets{SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX, SIZE_MAX};
     double cc[4 * kCarrLen];
@@ -3541,10 +3640,8 @@ int csx_stage_commit_many(csx_ctx* c, int n, const csx_staged* const* sts, int t
             c->bprep = true;
             FitSet f = st.f;
             radial_of(f, pd);
-            f.first_tile = c->bntiles_total;
             c->bntiles_total += st.ntiles;
             c->bsets.push_back(f);
-            c->bntiles.push_back(st.ntiles);
             c->bpend.push_back(pd);
             continue;
         }
@@ -3559,10 +3656,8 @@ int csx_stage_commit_many(csx_ctx* c, int n, const csx_staged* const* sts, int t
         pd.off_iso = at(st.pd.off_iso);
         FitSet f = st.f;
         radial_of(f, pd);
-        f.first_tile = c->bntiles_total;
         c->bntiles_total += st.ntiles;
         c->bsets.push_back(f);
-        c->bntiles.push_back(st.ntiles);
         c->bpend.push_back(pd);
     }
     return CSX_OK;
@@ -3612,10 +3707,20 @@ int csx_fit_batch_run(csx_ctx* c, int precision, double* h_sums, int64_t* h_cnts
 // the device addresses of every set's tables filled in; one H2D copy on the context's stream
 // (or a node of the round's graph).  Returns the device addresses of the records, of the flat
 // tile list (written on the device by k_prep_sets) and of the tile counts.
-static int batch_upload(csx_ctx* c, const FitSet** d_sets, const int2** d_tiles, const int** d_ntiles,
+static int batch_upload(csx_ctx* c, int precision, int* n_groups, const FitSet** d_sets, const int2** d_tiles, const int** d_ntiles,
                         size_t* bytes = nullptr) {
     const int nsets = (int)c->bsets.size();
-    const int ntiles = c->bntiles_total;
+    // the sets' workgroups in the launch's precision
+    int ntiles = 0;
+    c->bntiles.resize(nsets);
+    for (int i = 0; i < nsets; ++i) {
+        FitSet& f = c->bsets[i];
+        f.cov = fit_cover(f, kind_of(f.d.s.combo_key), precision);
+        f.first_tile = ntiles;
+        c->bntiles[i] = f.cov.total;
+        ntiles += f.cov.total;
+    }
+    *n_groups = ntiles;
     auto al = [](size_t o) { return (o + 255) & ~size_t(255); };
     if (c->brblock0.size() != (size_t)nsets + 1) return fail(c, CSX_E_STATE, "batch radial plan out of step");
     const size_t o_sets = al(c->barena.size);
@@ -3753,17 +3858,18 @@ int csx_fit_batch_launch(csx_ctx* c, int precision) {
     if (nsets == 0) return fail(c, CSX_E_STATE, "empty batch");
     precision = effective_precision(c->bsets[0].d.s.combo_key, precision);
     HIPCHK(c, hipSetDevice(c->device));
-    const int ntiles = c->bntiles_total;
+    int ntiles = 0;
     const FitSet* d_sets;
     const int2* d_tiles;
     const int* d_ntiles;
     size_t bytes = 0;
-    if (int rc = batch_upload(c, &d_sets, &d_tiles, &d_ntiles, c->use_graph ? &bytes : nullptr)) return rc;
+    if (int rc = batch_upload(c, precision, &ntiles, &d_sets, &d_tiles, &d_ntiles, c->use_graph ? &bytes : nullptr))
+        return rc;
     HIPCHK(c, c->bpart_d.ensure(ntiles * sizeof(TileSum)));
     HIPCHK(c, c->bsums_d.ensure(nsets * sizeof(SetSum)));
     HIPCHK(c, c->bres.reserve(nsets * sizeof(SetSum)));
     const int kind = kind_of(c->bsets[0].d.s.combo_key);
-    const int variant = c->tune_force >= 0 ? c->tune_force : tune_variant(kind, tune_size_class(ntiles, nsets));
+    const int variant = c->tune_force >= 0 ? c->tune_force : tune_variant(kind, tune_size_class(c->bntiles_total, nsets));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     if (c->use_graph) {
         const void* fn = nullptr;
@@ -3876,11 +3982,11 @@ extern "C" int csx_render_batch_run(csx_ctx* c, int precision) {
     for (const FitSet& f : c->bsets) {
         if (f.h != f.d.s.ymax - f.d.s.ymin) return fail(c, CSX_E_ARG, "a batched image must cover its whole grid");
     }
-    const int ntiles = c->bntiles_total;
+    int ntiles = 0;
     const FitSet* d_sets;
     const int2* d_tiles;
     const int* d_ntiles;
-    if (int rc = batch_upload(c, &d_sets, &d_tiles, &d_ntiles)) return rc;
+    if (int rc = batch_upload(c, precision, &ntiles, &d_sets, &d_tiles, &d_ntiles)) return rc;
     const int kind = kind_of(c->bsets[0].d.s.combo_key);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     hipLaunchKernelGGL(k_prep_sets, dim3(nsets), dim3(kPrepBlock), 0, c->stream, const_cast<FitSet*>(d_sets), nsets,
