@@ -325,10 +325,10 @@ __device__ __forceinline__ int wave_sum_i(int v) {
 
 // Relative error bounds of the two pair loops' sums, used by the conditioning guard.  FP32
 // loop: an exponent e carries ~7 ulp relative error plus the FP32 direction error of the
-// angular part, about 1e-5 of a term at the 2^-32 cut.  Precise loop: the FP32 exp2 of the
-// fraction (1 ulp), its conversion and the polynomial (2.4e-11 of y^2): 5e-7 with margin.
+// angular part, about 1e-5 of a term at the 2^-32 cut.  Precise loop: the angle polynomial
+// (2.4e-11 of y^2, times 22 at the cut) and exp2's (5.5e-11): 6e-10, 2e-9 with margin.
 constexpr double kRelErrFP32 = 1.0e-5;
-constexpr double kRelErrPrecise = 5.0e-7;
+constexpr double kRelErrPrecise = 2.0e-9;
 
 // |q^.u| above this can put the reference's FP64 cosine above 1, where its acos mapping
 // returns pi (Source/sc_calc_generic_gpu.cu:31): such pairs take the FP64 formula.
@@ -507,12 +507,29 @@ __device__ __forceinline__ double acos2_over_x(double x) {
     return p;
 }
 
-// 2^e for e <= 0 in FP64 exponent arithmetic with an FP32 exp2 of the fraction: relative
-// error about 1 ulp of FP32 whatever |e| (the FP32 loop's error grows with |e|).
-__device__ __forceinline__ double exp2_split(double e) {
+// 2^e for e <= 0 in FP64: 2^n times a degree-7 polynomial of the fraction |f| <= 1/2 (the
+// Chebyshev-node interpolant of 2^f, max relative error 5.5e-11).  FP64 FMAs issue at the rate
+// of FP32 ones here, so this costs what an FP32 exp2 with its two conversions does, and takes
+// the loop's error from 1e-7 to 1e-9: of the BCT cylinder patterns' pixels only those whose
+// structure factor cancels to 1e-4 of its terms are left to the FP64 re-sum, not to 1e-2.
+__device__ __forceinline__ double exp2_poly(double e) {
     const double n = rint(e);
-    const float f = (float)(e - n);  // |f| <= 1/2
-    return (double)ldexpf(__builtin_amdgcn_exp2f(f), (int)fmax(n, -200.0));
+    const double f = e - n;
+    double p = 1.53037004859714084e-05;
+    p = fma(p, f, 1.54697292255420087e-04);
+    p = fma(p, f, 1.33334784747766088e-03);
+    p = fma(p, f, 9.61802561323394332e-03);
+    p = fma(p, f, 5.55041090632442738e-02);
+    p = fma(p, f, 2.40226512134987719e-01);
+    p = fma(p, f, 6.93147180556833109e-01);
+    p = fma(p, f, 9.99999999959562902e-01);
+    return ldexp(p, (int)fmax(n, -1100.0));
+}
+// sqrt(x) for x >= 0 to 1e-13 relative: an FP32 reciprocal square root and one Newton step.
+__device__ __forceinline__ double sqrt_nr(double x) {
+    const double r = (double)__builtin_amdgcn_rsqf(fmaxf((float)x, 1.0e-30f));
+    const double y = x * r;
+    return fma(0.5 * r, fma(-y, y, x), y);
 }
 
 // Per-pixel constants of the precise pair loop.
@@ -539,11 +556,11 @@ __device__ __forceinline__ void pair_sum64(const PairRec64* __restrict__ prg, in
         const double t = L.q - (double)P.qh;
         const double r = (t * L.kr) * t;
         const double e1 = fma(L.kp, y2, r);
-        double w = exp2_split(e1);
+        double w = exp2_poly(e1);
         if constexpr (TWO) {
             // partner at pi - y: e2 = e1 + kp*pi*(pi - 2y)
-            const double y = (double)__builtin_amdgcn_sqrtf((float)y2);
-            w += exp2_split(fma(L.kp * kPi, kPi - 2.0 * y, e1));
+            const double y = sqrt_nr(y2);
+            w += exp2_poly(fma(L.kp * kPi, kPi - 2.0 * y, e1));
         }
         if constexpr (CHECK) {
             const bool fl = c > (double)kNearOne;
@@ -555,10 +572,10 @@ __device__ __forceinline__ void pair_sum64(const PairRec64* __restrict__ prg, in
                     const double yy = xx * acos2_over_x(xx);
                     const double tt = L.q - (double)P.qh;
                     const double ee = fma(L.kp, yy, (tt * L.kr) * tt);
-                    w = exp2_split(ee);
+                    w = exp2_poly(ee);
                     if constexpr (TWO) {
-                        const double y = (double)__builtin_amdgcn_sqrtf((float)yy);
-                        w += exp2_split(fma(L.kp * kPi, kPi - 2.0 * y, ee));
+                        const double y = sqrt_nr(yy);
+                        w += exp2_poly(fma(L.kp * kPi, kPi - 2.0 * y, ee));
                     }
                 }
             }
@@ -1261,16 +1278,19 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 const double pt = rv ? rv->pq : pq_cyl_transverse(d, q);
                 const double fr = rv ? rv->fq : fq_cyl_radial(d, q);
                 const double x = k ? -qx : qx, y = k ? -qy : qy;
-                double pl, fl;
-                switch (s.orcase) {
-                case 0:
-                    cyl_long_both(d, q, sqrt(s.cosphi * x * x + s.sinphi * y * y + 0.000000001),
-                                  x * s.cosphi * s.sintheta, y * s.sinphi * s.sintheta, pl, fl);
-                    break;
-                case 1: cyl_long_both(d, q, fabs(x), x, 0, pl, fl); break;
-                case 2: cyl_long_both(d, q, fabs(y), 0, y, pl, fl); break;
-                default: cyl_long_both(d, q, q, x, y, pl, fl); break;
+                double pl, fl, lim = q, xs = x, ys = y;
+                if (s.orcase == 0) {
+                    lim = sqrt(s.cosphi * x * x + s.sinphi * y * y + 0.000000001);
+                    xs = x * s.cosphi * s.sintheta;
+                    ys = y * s.sinphi * s.sintheta;
+                } else if (s.orcase == 1) {
+                    lim = fabs(x);
+                    ys = 0;
+                } else if (s.orcase == 2) {
+                    lim = fabs(y);
+                    xs = 0;
                 }
+                cyl_long_both<PREC == CSX_PREC_MIXED>(d, q, lim, xs, ys, pl, fl);
                 pq = pl * pt;
                 fq = fl * fr;
             }
@@ -2437,6 +2457,10 @@ void set_consts(DevSet& d) {
         d.cyl_g0 = csx::ref_gamma(zr + 1);
         d.cyl_g1 = csx::ref_gamma(zr - 1 / 2.0);
         d.cyl_g2 = csx::ref_gamma(zr - 3 / 2.0);
+        const double zl = (1 - s.sigmal * s.sigmal) / (s.sigmal * s.sigmal);
+        d.cyl_zl1 = zl - 1;
+        d.cyl_rc = 1 / (2.0 * zl * (zl - 1));
+        d.cyl_ll = s.length / (zl + 1);
     }
 }
 
@@ -2800,8 +2824,9 @@ static void launch_radial(const DevSet& d, const csx_grid& g, Radial* rtab, hipS
     }
 }
 
-// Blocks of the fix pass (one wave each; the pass steps through its queue).
-constexpr int kFixBlocks = 256;
+// Blocks of the fix pass (one wave each; the pass steps through its queue): one wave per SIMD
+// of the chip.
+constexpr int kFixBlocks = 1024;
 
 // ev: null, or two events recorded around the per-pixel kernel (the hot pass when two).
 template <int K, int P>

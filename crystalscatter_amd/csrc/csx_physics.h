@@ -88,6 +88,8 @@ struct DevSet {
     // Gamma(zr+1), Gamma(zr-1/2), Gamma(zr-3/2) of the transverse cylinder <F>^2 (zr from
     // sigma): per-set constants, evaluated once on the host with the reference's Gamma.
     double cyl_g0, cyl_g1, cyl_g2;
+    // z_L - 1, 1/(2 z_L (z_L - 1)) and L/(z_L + 1) of the rod factor's fast form (rod_p_fast)
+    double cyl_zl1, cyl_rc, cyl_ll;
     // Orientation quadrature of Gaussian-distributed cylinders in physics mode (built at
     // upload, see csx_device.hip): kCqDelta Gauss-Legendre polar nodes (cos, sin, weight),
     // kCqPsi/2 azimuth nodes t = cos(psi) of the midpoint rule on [0, pi], and the
@@ -136,32 +138,31 @@ __device__ __forceinline__ void pixel_q(const csx_scalars& s, int ihex, int i, d
     }
 }
 
-// Power series sum_n c[n] x^(2n) with the reference's exit rule (relative change < 1e-4),
-// the power built as (xn*x)*x.
-__device__ __forceinline__ double series_x2(const double* c, double x, int nmax) {
+// Power series sum_n c[n] x^(2n) with the reference's exit rule (relative change < 1e-4), the
+// power built as (xn*x)*x.  The rule |(sum - old)/sum| < 1e-4 is tested as |sum - old| <
+// 1e-4 |sum| (the same but for a rounding of the quotient onto the bound itself; zero, infinite
+// and NaN sums compare alike): the division took as long as the rest of the term.  Four
+// coefficients per trip, read wave-uniformly; nmax is a multiple of 4 below kCarrLen.
+__device__ __forceinline__ double series_x2(const double* cg, double x, int nmax) {
+    const auto c = (const __attribute__((address_space(4))) double*)cg;
     double sum = 1.0, old = 0.0, xn = 1.0;
-    for (int n = 1; n <= nmax; ++n) {
-        xn = xn * x * x;
-        sum = sum + c[n] * xn;
-        const double d = fabs((sum - old) / sum);
-        if (d < 0.0001) break;
-        old = sum;
+    bool go = true;
+    for (int n = 1; go && n <= nmax; n += 4) {
+        const double cc[4] = {c[n], c[n + 1], c[n + 2], c[n + 3]};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!go) break;
+            xn = xn * x * x;
+            sum = sum + cc[j] * xn;
+            go = !(fabs(sum - old) < 0.0001 * fabs(sum));
+            old = sum;
+        }
     }
     return sum;
 }
 
 // Same series in the longitudinal projection p = qxs+qys: the power is built as (xn*p)*p.
-__device__ __forceinline__ double series_proj(const double* c, double p, int nmax) {
-    double sum = 1.0, old = 0.0, xn = 1.0;
-    for (int n = 1; n <= nmax; ++n) {
-        xn = xn * p * p;
-        sum += c[n] * xn;
-        const double d = fabs((sum - old) / sum);
-        if (d < 0.0001) break;
-        old = sum;
-    }
-    return sum;
-}
+__device__ __forceinline__ double series_proj(const double* c, double p, int nmax) { return series_x2(c, p, nmax); }
 
 __device__ inline double pq_sphere(const DevSet& d, double q) {
     const csx_scalars& s = d.s;
@@ -376,8 +377,18 @@ __device__ inline double fq_cyl_zdir(const DevSet& d, double limql, double qxs, 
     return fq_cyl_long(d, limql, qxs, qys) * fq_cyl_radial(d, q);
 }
 
-// pq_cyl_long_zdir and fq_cyl_long at one pixel: the same values, with the rod average
-// evaluated once when both take it at the same argument (z_L agrees unless sigma_L = 1).
+// rod_p from the set's constants, for the mixed path: the power by exp and log, one division.
+// On the line where the projection vanishes the power is exactly 1, as rod_p's.
+__device__ __forceinline__ double rod_p_fast(const DevSet& d, double p) {
+    const double arg = p * d.cyl_ll, a2 = arg * arg;
+    const double lb = log(1.0 + 4 * a2);
+    return d.cyl_rc * (1 - cos(d.cyl_zl1 * atan(2.0 * arg)) * exp(-0.5 * d.cyl_zl1 * lb)) / a2;
+}
+
+// pq_cyl_long_zdir and fq_cyl_long at one pixel: the same values (FAST: to rounding), with the
+// rod average evaluated once when both take it at the same argument (z_L agrees unless
+// sigma_L = 1).
+template <bool FAST>
 __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, double qxs, double qys, double& pl,
                                      double& fl) {
     const csx_scalars& s = d.s;
@@ -391,10 +402,11 @@ __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, do
     const double zlf = (1 - sqd(s.sigmal)) / sqd(s.sigmal);
     const double zlp = s.sigmal == 1.0 ? 0.000000001 : zlf;
     const bool same = zlp == zlf;
+    const double p = qxs + qys + 0.000000001;
     double rod = 0.0;
-    if (!fser || (!pser && same)) rod = rod_p(zlf, (qxs + qys + 0.000000001) * s.length / (zlf + 1));
+    if (!fser || (!pser && same)) rod = FAST ? rod_p_fast(d, p) : rod_p(zlf, p * s.length / (zlf + 1));
     if (pser) pl = series_proj(carr_of<0>(d), qxs + qys, 120);
-    else pl = same ? rod : rod_p(zlp, (qxs + qys + 0.000000001) * s.length / (zlp + 1));
+    else pl = same ? rod : rod_p(zlp, p * s.length / (zlp + 1));
     fl = fser ? series_proj(carr_of<9>(d), qxs + qys, 120) : rod;
 }
 
