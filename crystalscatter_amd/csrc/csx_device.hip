@@ -525,6 +525,47 @@ __device__ __forceinline__ double exp2_poly(double e) {
     p = fma(p, f, 9.99999999959562902e-01);
     return ldexp(p, (int)fmax(n, -1100.0));
 }
+constexpr int kUnroll64 = 2;  // divides 4, the alignment of the segments
+// acos(c)^2 and exp2_poly for N arguments, step by step across them; each result equals
+// the single form's.
+template <int N>
+__device__ __forceinline__ void acos2_xn(const double* c, double* y2) {
+    constexpr double kC[12] = {5.8703930721466823e-04, -2.2269864280509148e-03, 4.3534013060061065e-03,
+                               -4.3610819883067170e-03, 3.8076579843268261e-03, 9.4124350172984761e-05,
+                               4.2622239283164089e-03, 1.0083515220786222e-02, 2.8579409148493790e-02,
+                               8.8888454904565387e-02, 3.3333334251157515e-01, 1.9999999999680802e+00};
+    double x[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        x[j] = 1.0 - c[j];
+        y2[j] = kC[0];
+    }
+#pragma unroll
+    for (int k = 1; k < 12; ++k)
+#pragma unroll
+        for (int j = 0; j < N; ++j) y2[j] = fma(y2[j], x[j], kC[k]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) y2[j] = x[j] * y2[j];
+}
+template <int N>
+__device__ __forceinline__ void exp2_poly_xn(const double* e, double* out) {
+    constexpr double kC[8] = {1.53037004859714084e-05, 1.54697292255420087e-04, 1.33334784747766088e-03,
+                              9.61802561323394332e-03, 5.55041090632442738e-02, 2.40226512134987719e-01,
+                              6.93147180556833109e-01, 9.99999999959562902e-01};
+    double n[N], f[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        n[j] = rint(e[j]);
+        f[j] = e[j] - n[j];
+        out[j] = kC[0];
+    }
+#pragma unroll
+    for (int k = 1; k < 8; ++k)
+#pragma unroll
+        for (int j = 0; j < N; ++j) out[j] = fma(out[j], f[j], kC[k]);
+#pragma unroll
+    for (int j = 0; j < N; ++j) out[j] = ldexp(out[j], (int)fmax(n[j], -1100.0));
+}
 // sqrt(x) for x >= 0 to 1e-13 relative: an FP32 reciprocal square root and one Newton step.
 __device__ __forceinline__ double sqrt_nr(double x) {
     const double r = (double)__builtin_amdgcn_rsqf(fmaxf((float)x, 1.0e-30f));
@@ -544,43 +585,84 @@ struct PixelConsts64 {
 template <bool PLANAR, bool TWO, bool CHECK, bool NEAR = false>
 __device__ __forceinline__ void pair_sum64(const PairRec64* __restrict__ prg, int p0, int p1, const PixelConsts64& L,
                                            double& acc, bool& flag, const NearCtx* nc = nullptr) {
+    // kUnroll64 pairs at a time, stage by stage, like pair_sum: one pair is a chain of about 40
+    // dependent FP64 operations, and small launches have one or two waves per SIMD to hide it.
+    // The next group's records are loaded while this one is evaluated: the table (48 KB) is
+    // larger than the scalar cache, so a group's loads take as long as its arithmetic.  The
+    // terms are added in pair order.
     constexpr double kPi = 3.14159265358979323846;
+    constexpr int U = kUnroll64;
     const auto pr = uniform_table(prg);
-    for (int p = p0; p < p1; ++p) {
-        const PairRec64 P = load_rec(pr, p);
-        double dt = fma(L.hy, P.uy, L.hx * P.ux);
-        if constexpr (!PLANAR) dt = fma(L.hz, P.uz, dt);
-        const double c = fabs(dt);
-        const double x = 1.0 - c;
-        const double y2 = x * acos2_over_x(x);
-        const double t = L.q - (double)P.qh;
-        const double r = (t * L.kr) * t;
-        const double e1 = fma(L.kp, y2, r);
-        double w = exp2_poly(e1);
+    struct Rec { double ux, uy, uz, A; float qh; };
+    auto load = [&](int i) {
+        Rec r;
+        r.ux = pr[i].ux;
+        r.uy = pr[i].uy;
+        if constexpr (!PLANAR) r.uz = pr[i].uz;
+        r.A = pr[i].A;
+        r.qh = pr[i].qh;
+        return r;
+    };
+    Rec N[U];
+    if (p0 < p1) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) N[j] = load(p0 + j);
+    }
+#pragma unroll 1
+    for (int p = p0; p < p1; p += U) {
+        Rec P[U];
+        double c[U], y2[U], e1[U], w[U];
+        const int pn = min(p + U, p1 - U);
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            P[j] = N[j];
+            N[j] = load(pn + j);
+        }
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            double dt = fma(L.hy, P[j].uy, L.hx * P[j].ux);
+            if constexpr (!PLANAR) dt = fma(L.hz, P[j].uz, dt);
+            c[j] = fabs(dt);
+        }
+        acos2_xn<U>(c, y2);
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const double t = L.q - (double)P[j].qh;
+            e1[j] = fma(L.kp, y2[j], (t * L.kr) * t);
+        }
+        exp2_poly_xn<U>(e1, w);
         if constexpr (TWO) {
             // partner at pi - y: e2 = e1 + kp*pi*(pi - 2y)
-            const double y = sqrt_nr(y2);
-            w += exp2_poly(fma(L.kp * kPi, kPi - 2.0 * y, e1));
+            double e2[U], w2[U];
+#pragma unroll
+            for (int j = 0; j < U; ++j) e2[j] = fma(L.kp * kPi, kPi - 2.0 * sqrt_nr(y2[j]), e1[j]);
+            exp2_poly_xn<U>(e2, w2);
+#pragma unroll
+            for (int j = 0; j < U; ++j) w[j] += w2[j];
         }
         if constexpr (CHECK) {
-            const bool fl = c > (double)kNearOne;
-            flag = flag || fl;
-            w = fl ? 0.0 : w;
-            if constexpr (NEAR) {
-                if (fl) {
-                    const double xx = near_pair_x<PLANAR>(*nc, P.ia);
-                    const double yy = xx * acos2_over_x(xx);
-                    const double tt = L.q - (double)P.qh;
-                    const double ee = fma(L.kp, yy, (tt * L.kr) * tt);
-                    w = exp2_poly(ee);
-                    if constexpr (TWO) {
-                        const double y = sqrt_nr(yy);
-                        w += exp2_poly(fma(L.kp * kPi, kPi - 2.0 * y, ee));
+#pragma unroll
+            for (int j = 0; j < U; ++j) {
+                const bool fl = c[j] > (double)kNearOne;
+                flag = flag || fl;
+                w[j] = fl ? 0.0 : w[j];
+                if constexpr (NEAR) {
+                    if (fl) {
+                        const double xx = near_pair_x<PLANAR>(*nc, pr[p + j].ia);
+                        const double yy = xx * acos2_over_x(xx);
+                        const double tt = L.q - (double)P[j].qh;
+                        const double ee = fma(L.kp, yy, (tt * L.kr) * tt);
+                        w[j] = exp2_poly(ee);
+                        if constexpr (TWO) {
+                            const double y = sqrt_nr(yy);
+                            w[j] += exp2_poly(fma(L.kp * kPi, kPi - 2.0 * y, ee));
+                        }
                     }
                 }
             }
         }
-        acc = fma(P.A, w, acc);
+#pragma unroll
+        for (int j = 0; j < U; ++j) acc = fma(P[j].A, w[j], acc);
     }
 }
 
@@ -1246,54 +1328,60 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
     if constexpr (!lattice_kind(KIND)) {
         v[0] = pixel_no_lattice<KIND>(d, qx, qy, q, rv);
     } else {
-        // P(q) and <F>^2 at the pixel (k = 0) or its mirror image (k = 1)
-        auto factors = [&](int k, double& pq, double& fq) {
+        // P(q) and <F>^2 at the pixel (0) and, for the oriented cylinder with NV = 2, at its
+        // mirror image (1)
+        constexpr int NV = KIND == K_BCT && PREC == CSX_PREC_MIXED ? 2 : 1;
+        double pq[NV], fqpq[NV];
+        auto factors = [&]() {
+            double fq[NV];
             if constexpr (KIND == K_FCC) {
                 if (rv) {
-                    pq = rv->pq;
-                    fq = rv->fq;
+                    pq[0] = rv->pq;
+                    fq[0] = rv->fq;
                 } else if constexpr (PREC == CSX_PREC_MIXED) {
-                    pq = pq_sphere_fast(d, q);
-                    fq = fq_sphere_fast(d, q);
+                    pq[0] = pq_sphere_fast(d, q);
+                    fq[0] = fq_sphere_fast(d, q);
                 } else {
-                    pq = pq_sphere(d, q);
-                    fq = fq_sphere(d, q);
+                    pq[0] = pq_sphere(d, q);
+                    fq[0] = fq_sphere(d, q);
                 }
             } else if constexpr (KIND == K_ISO_LAT) {
                 // calc_GENERIC, isotropic cylinders (Source/sc_gpu_generic.h:64-74: formpq and formfq
                 // of the cylinder at |q|) and homogeneous cubes (:295-302: formpq, and fq = pq)
                 if (rv) {
-                    pq = rv->pq;
-                    fq = rv->fq;
+                    pq[0] = rv->pq;
+                    fq[0] = rv->fq;
                 } else if (lattice_cube(s.combo_key)) {
-                    pq = pq_cube(d, q);
-                    fq = pq;
+                    pq[0] = pq_cube(d, q);
+                    fq[0] = pq[0];
                 } else {
-                    pq = pq_cyl_long_iso(d, q) * pq_cyl_transverse(d, q);
-                    fq = fq_cyl_long_iso(d, q) * fq_cyl_radial(d, q);
+                    pq[0] = pq_cyl_long_iso(d, q) * pq_cyl_transverse(d, q);
+                    fq[0] = fq_cyl_long_iso(d, q) * fq_cyl_radial(d, q);
                 }
             } else {
                 // the transverse P(q) and the radial factor of <F>^2 depend on |q| only: from the
                 // radial table when there is one (the same functions of the same |q|)
                 const double pt = rv ? rv->pq : pq_cyl_transverse(d, q);
                 const double fr = rv ? rv->fq : fq_cyl_radial(d, q);
-                const double x = k ? -qx : qx, y = k ? -qy : qy;
-                double pl, fl, lim = q, xs = x, ys = y;
+                double pl[NV], fl[NV], lim = q, xs = qx, ys = qy;
                 if (s.orcase == 0) {
-                    lim = sqrt(s.cosphi * x * x + s.sinphi * y * y + 0.000000001);
-                    xs = x * s.cosphi * s.sintheta;
-                    ys = y * s.sinphi * s.sintheta;
+                    lim = sqrt(s.cosphi * qx * qx + s.sinphi * qy * qy + 0.000000001);
+                    xs = qx * s.cosphi * s.sintheta;
+                    ys = qy * s.sinphi * s.sintheta;
                 } else if (s.orcase == 1) {
-                    lim = fabs(x);
+                    lim = fabs(qx);
                     ys = 0;
                 } else if (s.orcase == 2) {
-                    lim = fabs(y);
+                    lim = fabs(qy);
                     xs = 0;
                 }
-                cyl_long_both<PREC == CSX_PREC_MIXED>(d, q, lim, xs, ys, pl, fl);
-                pq = pl * pt;
-                fq = fl * fr;
+                cyl_long_both<NV, PREC == CSX_PREC_MIXED>(d, q, lim, xs, ys, pl, fl);
+                for (int k = 0; k < NV; ++k) {
+                    pq[k] = pl[k] * pt;
+                    fq[k] = fl[k] * fr;
+                }
             }
+            for (int k = 0; k < NV; ++k) fqpq[k] = fq[k] / pq[k];
         };
         double width = 1;
         if (s.dsch) width = 4.0 / s.domainsize;
@@ -1302,14 +1390,11 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
         double inten, radint;
         const double dwe = rv ? rv->dwe : exp(-s.dwfactor * q * q);
         // the factors follow the peak sum, so that they do not occupy registers during it
-        constexpr int NV = KIND == K_BCT && PREC == CSX_PREC_MIXED ? 2 : 1;
-        double pq[NV], fqpq[NV], inten2;
+        double inten2;
         if constexpr (PREC == CSX_PREC_REF64) {
             lattice_ref64(d, qx, qy, qz, q, width, inten, radint);
             inten2 = inten;
-            double fq;
-            factors(0, pq[0], fq);
-            fqpq[0] = fq / pq[0];
+            factors();
         } else {
             bool need_exact = false;
             double dropped = 0.0;
@@ -1337,17 +1422,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                             : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, stats);
             }
             radint = (s.iso != 0) ? iso_mixed(d, q) : 0.0;
-#pragma unroll
-            for (int k = 0; k < NV; ++k) {
-                if (k == 0 || mir) {
-                    double fq;
-                    factors(k, pq[k], fq);
-                    fqpq[k] = fq / pq[k];
-                } else {
-                    pq[k] = pq[0];
-                    fqpq[k] = fqpq[0];
-                }
-            }
+            factors();
             // Conditioning guard.  szq = 1 + B - (fq/pq)*dwe with B = (fq/pq)*(2*pi*I/V)*dwe.
             // The peak sum I carries up to kRelErrFP32 (FP32 loop) or kRelErrPrecise (precise
             // loop) relative error plus this lane's dropped mass; szq amplifies an error of I
@@ -1359,7 +1434,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
             auto loose = [&](double I, double rel) {
                 bool any = false;
 #pragma unroll
-                for (int k = 0; k < NV; ++k) {
+                for (int k = 0; k < (mir ? NV : 1); ++k) {
                     const double bs = fqpq[k] * d.two_pi_over_v * dwe;
                     const double szq_est = 1 + fqpq[k] * (I * d.two_pi_over_v - 1) * dwe;
                     const double dsz = fabs(bs) * (rel * fabs(I) + dropped * inv_hpw);
@@ -1376,12 +1451,15 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                               (W.near ? 1 : 0) | (need_exact ? 2 : 0) | (mir ? 8 : 0), 0};
                 inten2 = inten;
             } else {
-                if (__ballot(want2)) {
-                    if (want2) need_q(s, P3);
-                    coop_window_sum64<kPrecise>(d, W, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want2, inten);
-                    if (stats && want2) atomicAdd(&stats[1], 1ull);
+                // straight to the full sum where the dropped mass alone is too coarse
+                bool want3 = need_exact || (want2 && loose(inten, 1.0e-13));
+                const bool window = want2 && !want3;
+                if (__ballot(window)) {
+                    if (window) need_q(s, P3);
+                    coop_window_sum64<kPrecise>(d, W, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, window, inten);
+                    if (stats && window) atomicAdd(&stats[1], 1ull);
                 }
-                const bool want3 = need_exact || (want2 && loose(inten, 1.0e-13));
+                want3 = want3 || (window && loose(inten, 1.0e-13));
                 inten2 = inten;
                 if (__ballot(want3)) {
                     if (want3) need_q(s, P3);
@@ -1430,7 +1508,11 @@ __device__ __forceinline__ void tile_pixel(int& px, int& py) {
 // Plain: one 16x16 tile each.  With mirror images (x0 = -x1, y0 = -y1): tiles over the rows
 // i < 0 only, each lane's value serving (ihex, i) and (-ihex, -i); the row i = 0 left of and
 // at the axis, and the column ihex = x0 below it (whose mirror images lie outside the block),
-// follow as workgroups of 256 consecutive pixels.  That is 2 z^2 + 2 z of 4 z^2 pixels.
+// follow, 16 consecutive pixels per wave (64 of them in a row have a |q| range, and so a pair
+// loop, several times a tile's, and were the tail of the whole launch).  That is 2 z^2 + 2 z
+// of 4 z^2 pixels.
+constexpr int kStrip = 16;                          // strip pixels per wave
+constexpr int kStripBlock = kStrip * (kBlock / 64); // and per workgroup
 struct Cover {
     int32_t x0, x1, y0, y1;
     int32_t mirror, tiles_x, main, total;  // main: 16x16 tiles; total: workgroups
@@ -1439,7 +1521,7 @@ __host__ __device__ inline Cover make_cover(int x0, int x1, int y0, int y1, bool
     Cover c{x0, x1, y0, y1, mirror ? 1 : 0, 0, 0, 0};
     c.tiles_x = (x1 - x0 + kTile - 1) / kTile;
     c.main = c.tiles_x * (((mirror ? -y0 : y1 - y0) + kTile - 1) / kTile);
-    c.total = c.main + (mirror ? (x1 + y1 + kBlock - 1) / kBlock : 0);
+    c.total = c.main + (mirror ? (x1 + y1 + kStripBlock - 1) / kStripBlock : 0);
     return c;
 }
 struct CoverPix {
@@ -1459,8 +1541,9 @@ __device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t) {
         p.i = min(i, ylim - 1);
         p.mir = c.mirror && p.in && ihex > c.x0 && i > c.y0;
     } else {
-        const int n = (t - c.main) * kBlock + (int)threadIdx.x;
-        p.in = n < c.x1 + c.y1;
+        const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+        const int n = (t - c.main) * kStripBlock + w * kStrip + min(lane, kStrip - 1);
+        p.in = n < c.x1 + c.y1 && lane < kStrip;
         const int k = min(n, c.x1 + c.y1 - 1);
         const bool row = k <= c.x1;
         p.ihex = row ? c.x0 + k : c.x0;
@@ -1473,7 +1556,7 @@ __device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t) {
 // midpoint grid, when every reflection has its Friedel partner in the list.
 inline bool mirror_set(const DevSet& d, int kind, int precision, int x0, int x1, int y0, int y1) {
     return lattice_kind(kind) && precision == CSX_PREC_MIXED && d.nsingle == 0 && !d.s.centerbeam && !d.s.use1d &&
-           x1 > 0 && y1 > 0 && x0 == -x1 && y0 == -y1;
+           !(kind == K_BCT && d.s.sigmal == 1.0) && x1 > 0 && y1 > 0 && x0 == -x1 && y0 == -y1;
 }
 
 // Kinds whose form factors depend on |q| only.
@@ -1758,7 +1841,7 @@ __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __re
             if (!fit_masked(s, f.m, f.data, f.w, x, y)) {
                 const double dv = f.data[idx];
                 if (v[k] > 0 && dv > 0) {
-                    const double a = log(v[k]) / log(10.) - log(dv) / log(10.);
+                    const double a = (log(v[k]) - log(dv)) * 0.43429448190325182765;  // log10(v / dv)
                     tk = a * a;
                 }
             }

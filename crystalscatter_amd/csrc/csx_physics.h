@@ -141,22 +141,27 @@ __device__ __forceinline__ void pixel_q(const csx_scalars& s, int ihex, int i, d
 // Power series sum_n c[n] x^(2n) with the reference's exit rule (relative change < 1e-4), the
 // power built as (xn*x)*x.  The rule |(sum - old)/sum| < 1e-4 is tested as |sum - old| <
 // 1e-4 |sum| (the same but for a rounding of the quotient onto the bound itself; zero, infinite
-// and NaN sums compare alike): the division took as long as the rest of the term.  Four
-// coefficients per trip, read wave-uniformly; nmax is a multiple of 4 below kCarrLen.
+// and NaN sums compare alike): the division took as long as the rest of the term.  Four terms
+// per trip, taken together with their exits picked afterwards (a branch per term costs more
+// than the terms past the exit); the coefficients are read wave-uniformly.  nmax is a multiple
+// of 4 below kCarrLen.
 __device__ __forceinline__ double series_x2(const double* cg, double x, int nmax) {
     const auto c = (const __attribute__((address_space(4))) double*)cg;
     double sum = 1.0, old = 0.0, xn = 1.0;
     bool go = true;
+#pragma unroll 1
     for (int n = 1; go && n <= nmax; n += 4) {
-        const double cc[4] = {c[n], c[n + 1], c[n + 2], c[n + 3]};
+        double s[4];
+        bool done[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            if (!go) break;
             xn = xn * x * x;
-            sum = sum + cc[j] * xn;
-            go = !(fabs(sum - old) < 0.0001 * fabs(sum));
-            old = sum;
+            s[j] = (j ? s[j - 1] : sum) + c[n + j] * xn;
+            done[j] = fabs(s[j] - (j ? s[j - 1] : old)) < 0.0001 * fabs(s[j]);
         }
+        sum = done[0] ? s[0] : done[1] ? s[1] : done[2] ? s[2] : s[3];
+        old = s[3];
+        go = !(done[0] || done[1] || done[2] || done[3]);
     }
     return sum;
 }
@@ -377,24 +382,42 @@ __device__ inline double fq_cyl_zdir(const DevSet& d, double limql, double qxs, 
     return fq_cyl_long(d, limql, qxs, qys) * fq_cyl_radial(d, q);
 }
 
-// rod_p from the set's constants, for the mixed path: the power by exp and log, one division.
-// On the line where the projection vanishes the power is exactly 1, as rod_p's.
-__device__ __forceinline__ double rod_p_fast(const DevSet& d, double p) {
-    const double arg = p * d.cyl_ll, a2 = arg * arg;
+// rod_p from the set's constants, for the mixed path, at the projection p + 1e-9 and, with two,
+// at its mirror image -p + 1e-9: the power by exp and log, one division.  On the line p = 0 the
+// power is exactly 1, as rod_p's.  The rod factor f is even, so f(-p + e) = f(p - e) =
+// f(p + e) - 2 e f'(p) + O(e^3), and with e = 1e-9 an FP32 slope leaves about 1e-13 of f: a
+// second evaluation, in a loop or inlined, took 70 registers or its own 250 operations.
+template <int NV>
+__device__ __forceinline__ void rod_p_fast(const DevSet& d, double p, double* out) {
+    const double arg = (p + 0.000000001) * d.cyl_ll, a2 = arg * arg;
     const double lb = log(1.0 + 4 * a2);
-    return d.cyl_rc * (1 - cos(d.cyl_zl1 * atan(2.0 * arg)) * exp(-0.5 * d.cyl_zl1 * lb)) / a2;
+    const double ph = d.cyl_zl1 * atan(2.0 * arg);
+    const double c = cos(ph), E = exp(-0.5 * d.cyl_zl1 * lb);
+    const double g = 1 - c * E;
+    const double ia2 = 1 / a2;
+    out[0] = d.cyl_rc * g * ia2;
+    if constexpr (NV > 1) {
+        // f = rc g / a^2, g = 1 - cos(ph) E: g' = E ph' (sin(ph) + 2 a cos(ph)), ph' = 2 n / (1 + 4 a^2)
+        const float a = (float)arg;
+        const float dph = (float)(2.0 * d.cyl_zl1) * __builtin_amdgcn_rcpf(__builtin_fmaf(4.0f * a, a, 1.0f));
+        const float sn = __builtin_amdgcn_sinf(__builtin_amdgcn_fractf((float)(ph * 0.15915494309189535)));
+        const float gp = (float)E * dph * __builtin_fmaf(2.0f * a, (float)c, sn);
+        const float slope = gp - 2.0f * (float)g * __builtin_amdgcn_rcpf(a);
+        out[1] = out[0] - 2.0e-9 * d.cyl_ll * d.cyl_rc * ia2 * (double)slope;
+        if (p == 0.0) out[1] = out[0];
+    }
 }
 
 // pq_cyl_long_zdir and fq_cyl_long at one pixel: the same values (FAST: to rounding), with the
 // rod average evaluated once when both take it at the same argument (z_L agrees unless
-// sigma_L = 1).
-template <bool FAST>
-__device__ inline void cyl_long_both(const DevSet& d, double q, double limql, double qxs, double qys, double& pl,
-                                     double& fl) {
+// sigma_L = 1).  NV = 2 (sets with sigma_L != 1): also at the mirror image, whose series are
+// the same (even in the projection) and whose rod argument is -(qxs + qys) + 1e-9.
+template <int NV, bool FAST>
+__device__ inline void cyl_long_both(const DevSet& d, double q, double limql, double qxs, double qys, double* pl,
+                                     double* fl) {
     const csx_scalars& s = d.s;
     if (orc_cmp(s) == 4) {
-        pl = 1.0;
-        fl = 1.0;
+        for (int k = 0; k < NV; ++k) pl[k] = fl[k] = 1.0;
         return;
     }
     const bool pser = q < (0.6 * s.limq[0]);
@@ -402,12 +425,20 @@ __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, do
     const double zlf = (1 - sqd(s.sigmal)) / sqd(s.sigmal);
     const double zlp = s.sigmal == 1.0 ? 0.000000001 : zlf;
     const bool same = zlp == zlf;
-    const double p = qxs + qys + 0.000000001;
-    double rod = 0.0;
-    if (!fser || (!pser && same)) rod = FAST ? rod_p_fast(d, p) : rod_p(zlf, p * s.length / (zlf + 1));
-    if (pser) pl = series_proj(carr_of<0>(d), qxs + qys, 120);
-    else pl = same ? rod : rod_p(zlp, p * s.length / (zlp + 1));
-    fl = fser ? series_proj(carr_of<9>(d), qxs + qys, 120) : rod;
+    const double p = qxs + qys;
+    const double ps = pser ? series_proj(carr_of<0>(d), p, 120) : 0.0;
+    const double fs = fser ? series_proj(carr_of<9>(d), p, 120) : 0.0;
+    double rod[NV];
+    for (int k = 0; k < NV; ++k) rod[k] = 0.0;
+    if (!fser || (!pser && same)) {
+        if constexpr (FAST) rod_p_fast<NV>(d, p, rod);
+        else rod[0] = rod_p(zlf, (p + 0.000000001) * s.length / (zlf + 1));
+    }
+    for (int k = 0; k < NV; ++k) {
+        pl[k] = pser ? ps : rod[k];
+        fl[k] = fser ? fs : rod[k];
+    }
+    if (!pser && !same) pl[0] = rod_p(zlp, (p + 0.000000001) * s.length / (zlp + 1));
 }
 
 }  // namespace csx
