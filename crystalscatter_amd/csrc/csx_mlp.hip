@@ -11,13 +11,12 @@
 //   output  1 (linear)
 //
 // Precision: BF16 weights and activations on the matrix cores (v_mfma_f32_16x16x32_bf16),
-// FP32 accumulation, FP32 master weights and Adam state.  Every matrix product is one
-// "NT" kernel, C[m][n] = sum_k A[m][k] * B[n][k] with both operands k-contiguous:
-//   forward   Z_l  = H_{l-1} . W_l^T      A = H_{l-1} [M][K], B = W_l   [N][K] (out x in)
-//   backward  dH   = dZ_l . W_l          A = dZ_l [M][N],    B = W_l^T [K][N]
-//   weights   dW_l = dZ_l^T . H_{l-1}    A = dZ_l^T [N][M],  B = H_{l-1}^T [K][M], split over M
-// so the forward pass also stores H^T and the backward pass dZ^T (bf16), and each weight is
-// kept in bf16 in both orientations.  Per-sample buffers are sized for max_batch rows.
+// FP32 accumulation, FP32 master weights and Adam state.  One kernel takes kPM rows through the
+// whole network with their activations in one LDS tile (k_mlp: inference, or forward and
+// backward with Z kept in registers); for the weight gradients it also leaves H_{l-1}^T and
+// dZ_l^T (bf16) behind, and dW_l = dZ_l^T . H_{l-1} is one NT product over the rows for all
+// layers together (k_wgrad), whose split partials k_finish adds in a fixed order.  Each weight
+// is kept in bf16 in both orientations.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,6 +33,7 @@ namespace csm {
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kIn = CSX_MLP_IN_PAD;    // padded input width
@@ -42,9 +42,7 @@ constexpr int kH = CSX_MLP_HIDDEN;     // hidden width
 constexpr int kL = CSX_MLP_LAYERS;     // hidden layers
 constexpr int kNF = CSX_MLP_NFREQ;     // Fourier frequencies
 constexpr int kNP = CSX_MLP_NPAR;      // parameters per set
-constexpr int kBM = 128, kBN = 128, kBK = 64, kLd = kBK + 8;  // GEMM tile, LDS row stride (bf16)
-constexpr int kTp = kBN + 8;            // row stride (bf16) of the epilogue's output tile in LDS
-constexpr int kHeadRows = 64;           // rows per block of the output-layer kernels
+constexpr int kBM = 128;               // max_batch is rounded up to a multiple of this
 
 // Offsets of the FP32 master parameters (one buffer): hidden layer l has W_l [kH][in_l]
 // (out x in) then b_l [kH]; then the output weights w [kH] and bias.
@@ -57,10 +55,22 @@ constexpr int64_t kOutW = w_off(kL);
 constexpr int64_t kOutB = kOutW + kH;
 constexpr int64_t kNParams = kOutB + 1;
 
-__device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + __expf(-z)); }
+// Sigmoid from the hardware exp2 and reciprocal (1 ulp each): the activations are stored in
+// bf16, and an IEEE division here was a third of the inference's instructions.
+__device__ __forceinline__ float sigm(float z) {
+    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950409f * z));
+}
 __device__ __forceinline__ float silu_grad(float z) {
     const float s = sigm(z);
-    return s * (1.0f + z * (1.0f - s));
+    return s * __builtin_fmaf(z, 1.0f - s, 1.0f);
+}
+
+// Position of weight (row, k) of a [rows][K] matrix in its bf16 copy: MFMA A fragments of 16 rows
+// x 32 k one after the other, rows first, each as the 64 lanes hold it (lane row % 16 +
+// 16 (k % 32 / 8), 8 values), so a wave's fragment load is 1 KB in a row.  Row-major, it touched
+// 16 cache lines of which it used half.
+__host__ __device__ constexpr int frag_index(int row, int k, int rows) {
+    return ((k / 32) * (rows / 16) + row / 16) * 512 + ((row % 16) + 16 * (k % 32 / 8)) * 8 + k % 8;
 }
 
 // ---- input features ----------------------------------------------------------------
@@ -72,441 +82,459 @@ struct Features {
     float off[kNP], sc[kNP];
 };
 
-// Row i < n: parameters of set[i] (already normalised by the caller; an index outside
-// [0, nsets) is clamped, the host checks them), then sin and cos of the kNF phases; rows
-// n..mpad-1 are zero.  Writes X [mpad][kIn] and X^T [kIn][mpad].
-__global__ void __launch_bounds__(256) k_embed(int n, int mpad, int nsets, const float* __restrict__ par,
-                                               const int32_t* __restrict__ set, const float* __restrict__ q,
-                                               const Features ft, bf16* __restrict__ X, bf16* __restrict__ XT) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= mpad) return;
-    float v[kIn];
+// ---- the network over kPM rows ---------------------------------------------------------
+// NW waves; wave w owns 256 / NW consecutive features of every layer.  A layer is the product
+// W . H^T (D[feature][row]): the weights are the A operand, read straight from the bf16
+// [out][in] copies (L2-resident), the rows' activations the B operand, from LDS.  A lane then
+// holds four consecutive features of one row, so the epilogue writes 8 bytes where the other
+// orientation writes four 2-byte values.  The bias is the accumulators' initial value.
+// Bound: the vector unit -- per row 1024 SiLU values at about 46 cycles each per wave of 64
+// (exp2 and reciprocal at quarter rate) against 422 matrix cycles.  2.1 M rows of inference:
+// 1.22 ms (2.72 ms with H . W^T, IEEE divisions and row-major weights); with 8 waves 1.32 ms.
+// Training, 65,536 rows: 0.16 ms, its phases between barriers (4 waves at 2 per SIMD: 0.22 ms),
+// for the 11 launches and 0.38 ms of the layer-by-layer passes.
+constexpr int kPM = 64;        // rows per block
+constexpr int kInferWaves = 4, kTrainWaves = 8;
+constexpr int kPLd = kH + 8;   // LDS row stride (bf16): 16-byte aligned rows
+static_assert(kPM == 64 && kH == 256, "one lane per row");
+
+// Parameters of set[i] (already normalised by the caller; an index outside [0, nsets) is
+// clamped, the host checks them), then sin and cos of the kNF phases, then zeros; rows >= n are
+// zero.  Lane = row; each wave takes kNF / NW phases.  The phase is formed in turns.
+template <int NW>
+__device__ __forceinline__ void embed_rows(int r0, int n, int nsets, const float* __restrict__ par,
+                                           const int32_t* __restrict__ set, const float* __restrict__ q,
+                                           const Features& ft, bf16* act) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = r0 + lane;
+    const bool live = i < n;
+    float v[kNP];
 #pragma unroll
-    for (int k = 0; k < kIn; ++k) v[k] = 0.0f;
-    if (i < n) {
-        const float* p = par + (size_t)min(max(set[i], 0), nsets - 1) * kNP;  // clamped: never out of bounds
+    for (int k = 0; k < kNP; ++k) v[k] = 0.0f;
+    float qx = 0.0f, qy = 0.0f;
+    if (live) {
+        const float* pp = par + (size_t)min(max(set[i], 0), nsets - 1) * kNP;  // clamped: never out of bounds
 #pragma unroll
-        for (int k = 0; k < kNP; ++k) v[k] = p[k];
-        const float qx = q[2 * i], qy = q[2 * i + 1];
-        const float qa = sqrtf(qx * qx + qy * qy);
-#pragma unroll
-        for (int f = 0; f < kNF; ++f) {
-            const int j = ft.pidx[f];
-            float pv = 1.0f;  // constant indices only: v stays in registers
-#pragma unroll
-            for (int k = 0; k < kNP; ++k) pv = (k == j) ? ft.off[k] + ft.sc[k] * v[k] : pv;
-            float s, c;
-            sincosf(6.283185307f * (ft.f[f][0] * qx + ft.f[f][1] * qy) + ft.f[f][2] * qa * pv, &s, &c);
-            v[kNP + f] = s;
-            v[kNP + kNF + f] = c;
-        }
+        for (int k = 0; k < kNP; ++k) v[k] = pp[k];
+        qx = q[2 * (size_t)i];
+        qy = q[2 * (size_t)i + 1];
     }
-    bf16* row = X + (size_t)i * kIn;
+    uint32_t* row = reinterpret_cast<uint32_t*>(act + lane * kPLd);
+    auto pack = [](float a, float b) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 p = {(bf16)a, (bf16)b};
+        return __builtin_bit_cast(uint32_t, p);
+    };
+    static_assert(kNP % 2 == 0 && kNF % 8 == 0 && kIn % 2 == 0, "features in pairs");
+    if (wave == 0)
 #pragma unroll
-    for (int k = 0; k < kIn; k += 8) {
-        bf16x8 pk;
+        for (int k = 0; k < kNP; k += 2) row[k / 2] = pack(v[k], v[k + 1]);
+    const float qa = sqrtf(qx * qx + qy * qy) * 0.15915494309f;  // turns
+    constexpr int NF = kNF / NW;
+    float sn[NF], cs[NF];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) pk[j] = (bf16)v[k + j];
-        *(bf16x8*)(row + k) = pk;
+    for (int f0 = 0; f0 < NF; ++f0) {
+        const int f = wave * NF + f0;
+        const int j = ft.pidx[f];
+        float pv = 1.0f;
+#pragma unroll
+        for (int k = 0; k < kNP; ++k) pv = (k == j) ? ft.off[k] + ft.sc[k] * v[k] : pv;
+        const float turn =
+            __builtin_amdgcn_fractf((ft.f[f][0] * qx + ft.f[f][1] * qy) + ft.f[f][2] * qa * pv);
+        sn[f0] = live ? __builtin_amdgcn_sinf(turn) : 0.0f;
+        cs[f0] = live ? __builtin_amdgcn_cosf(turn) : 0.0f;
     }
 #pragma unroll
-    for (int k = 0; k < kIn; ++k) XT[(size_t)k * mpad + i] = (bf16)v[k];
+    for (int f0 = 0; f0 < NF; f0 += 2) {
+        row[(kNP + NF * wave + f0) / 2] = pack(sn[f0], sn[f0 + 1]);
+        row[(kNP + kNF + NF * wave + f0) / 2] = pack(cs[f0], cs[f0 + 1]);
+    }
+    for (int k = kUsed / 2 + wave; k < kIn / 2; k += NW) row[k] = 0u;
 }
 
-// ---- the NT matrix product with its epilogues ---------------------------------------
-enum Epi { EPI_FWD = 0, EPI_BWD = 1, EPI_PART = 2 };
-struct EpiArgs {
-    const float* bias;   // FWD: b_l
-    bf16* z;             // FWD: Z_l [M][N] out
-    bf16* h;             // FWD: H_l [M][N] out
-    bf16* ht;            // FWD: H_l^T [N][M] out
-    const bf16* zprev;   // BWD: Z_{l-1} [M][N]
-    bf16* dz;            // BWD: dZ_{l-1} [M][N] out
-    bf16* dzt;           // BWD: dZ_{l-1}^T [N][M] out
-    float* part;         // PART: partials [split][M][N]
-    int ldo;             // leading dimension of [M][N] outputs (N)
-    int ldt;             // leading dimension of the transposed outputs (M)
+// acc[i][j] += the wave's 16 NI features x kPM rows of W . act^T over k < K (W in fragment order,
+// kH rows).
+template <int K, int NI, bool PREFETCH>
+__device__ __forceinline__ void layer_product(const bf16* __restrict__ W, const bf16* act, int wn, f32x4 (&acc)[NI][4]) {
+    const int lane = threadIdx.x & 63, fr = lane & 15, fk = (lane >> 4) * 8;
+    const bf16* wp = W + (size_t)(wn / 16) * 512 + lane * 8;
+    if constexpr (PREFETCH) {
+        bf16x8 a[NI], an[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) a[i] = *(const bf16x8*)(wp + i * 512);
+#pragma unroll
+        for (int ks = 0; ks < K; ks += 32) {
+            if (ks + 32 < K)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) an[i] = *(const bf16x8*)(wp + ((ks / 32 + 1) * (kH / 16) + i) * 512);
+            bf16x8 b[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = *(const bf16x8*)&act[(j * 16 + fr) * kPLd + ks + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i) a[i] = an[i];
+        }
+    } else {
+        // training: half of the registers hold Z, no room for a second set of fragments
+#pragma unroll 1
+        for (int ks = 0; ks < K; ks += 32, wp += (kH / 16) * 512) {
+            bf16x8 a[NI], b[4];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) a[i] = *(const bf16x8*)(wp + i * 512);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = *(const bf16x8*)&act[(j * 16 + fr) * kPLd + ks + fk];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
+// Accumulator (i, j)[r] is feature wn + 16 i + 4 (lane / 16) + r of row 16 j + lane % 16.
+__device__ __forceinline__ int acc_feature(int wn, int i) { return wn + i * 16 + ((threadIdx.x & 63) >> 4) * 4; }
+__device__ __forceinline__ int acc_row(int j) { return j * 16 + (threadIdx.x & 15); }
+
+// The LDS tile's transpose to outT, a [ncol][kPM] matrix in fragment order (frag_index), which is
+// what k_wgrad's MFMAs take: a block's rows are contiguous (with all rows of a feature in a row, a
+// tile's 256 pieces lay 128 KB apart and shared a few memory channels).  A thread takes two
+// features and 2 / NW of the rows (b32 reads, conflict-free), one k octet of both in 32 bytes; with
+// SUM the columns' sums over those rows as well.
+// Partial sums per block of kPM rows: biases of the kL layers, output weights, output bias, loss.
+constexpr int kPartB = (kL + 1) * kH + 2;
+template <int NW, bool SUM>
+__device__ __forceinline__ void store_columns(const bf16* act, bf16* __restrict__ outT, int ncol,
+                                              float* __restrict__ sums) {
+    constexpr int R = 2 * kPM / NW;
+    const int c = (threadIdx.x & 127) * 2, h = (threadIdx.x >> 7) * R;
+    if (c >= ncol) return;
+    float s0 = 0.0f, s1 = 0.0f;
+#pragma unroll
+    for (int g = 0; g < R; g += 8) {
+        uint32_t x[8];
+        uint4 lo, hi;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = *(const uint32_t*)&act[(h + g + k) * kPLd + c];
+        uint32_t* lp = reinterpret_cast<uint32_t*>(&lo);
+        uint32_t* hp = reinterpret_cast<uint32_t*>(&hi);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            lp[k] = (x[2 * k] & 0xffffu) | (x[2 * k + 1] << 16);
+            hp[k] = (x[2 * k] >> 16) | (x[2 * k + 1] & 0xffff0000u);
+        }
+        if constexpr (SUM) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                s0 += __uint_as_float(x[k] << 16);
+                s1 += __uint_as_float(x[k] & 0xffff0000u);
+            }
+        }
+        *(uint4*)&outT[frag_index(c, h + g, ncol)] = lo;
+        *(uint4*)&outT[frag_index(c + 1, h + g, ncol)] = hi;
+    }
+    if constexpr (SUM) *(float2*)&sums[(threadIdx.x >> 7) * kH + c] = make_float2(s0, s1);
+}
+
+// Training outputs of k_mlp.
+struct TrainArgs {
+    const float* tgt;     // targets
+    bf16* xt;             // X^T, H_l^T, dZ_l^T: per block of kPM rows [features][kPM], fragments
+    bf16* ht[kL - 1];
+    bf16* dzt[kL];
+    const bf16* wtb;      // weights [in][out]
+    float* part;          // [blocks][kPartB]
 };
 
-// Grid (M/128, N/128, splits); 256 threads, 4 waves in 2x2, each wave a 64x64 block of
-// 4x4 MFMA tiles.  Requires M, N multiples of 128, K and kchunk multiples of 64, lda/ldb
-// multiples of 8 (checked by the host).
-// Row phase of the epilogue: the 128x128 bf16 tile T (row stride kTp) to out[m][n] rows with
-// 16-byte stores (out row stride ld).
-__device__ __forceinline__ void tile_store_rows(const bf16* T, bf16* __restrict__ out, int ld, int tm, int tn) {
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-        const int id = threadIdx.x + 256 * it;
-        const int row = id >> 4, c8 = (id & 15) * 8;
-        *(uint4*)&out[(size_t)(tm + row) * ld + tn + c8] = *(const uint4*)&T[row * kTp + c8];
-    }
-}
-// Column phase: the transpose of T to outT[n][m] (row stride ldt), 8 rows per 16-byte store;
-// consecutive threads take consecutive columns (conflict-free LDS reads).
-__device__ __forceinline__ void tile_store_cols(const bf16* T, bf16* __restrict__ outT, int ldt, int tm, int tn) {
-#pragma unroll
-    for (int it = 0; it < 8; ++it) {
-        const int id = threadIdx.x + 256 * it;
-        const int col = id & 127, m8 = (id >> 7) * 8;
-        bf16x8 pk;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) pk[k] = T[(m8 + k) * kTp + col];
-        *(bf16x8*)&outT[(size_t)(tn + col) * ldt + tm + m8] = pk;
-    }
-}
-
-template <int EPI>
-__global__ void __launch_bounds__(256) k_gemm_nt(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
-                                                 int ldb, int K, int kchunk, EpiArgs ep) {
-    // operand tiles during the main loop, the output tile (128 x kTp bf16) in the epilogue
-    __shared__ __attribute__((aligned(16))) bf16 smem[2 * kBM * kLd];
-    static_assert(kBM * kTp <= 2 * kBM * kLd, "epilogue tile must fit in the operand tiles");
-    bf16* sA = smem;
-    bf16* sB = smem + kBM * kLd;
-    bf16* T = smem;
-    const int tm = blockIdx.x * kBM, tn = blockIdx.y * kBN;
-    const int k0 = blockIdx.z * kchunk, k1 = min(K, k0 + kchunk);
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
-    const int fr = lane & 15, fk = (lane >> 4) * 8;  // fragment row, k offset
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int kk = k0; kk < k1; kk += kBK) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = t + r * 256;
-            const int row = idx >> 3, c8 = (idx & 7) * 8;
-            *(uint4*)&sA[row * kLd + c8] = *(const uint4*)&A[(size_t)(tm + row) * lda + kk + c8];
-            *(uint4*)&sB[row * kLd + c8] = *(const uint4*)&B[(size_t)(tn + row) * ldb + kk + c8];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < kBK; ks += 32) {
-            bf16x8 af[4], bfg[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = *(const bf16x8*)&sA[(wm + i * 16 + fr) * kLd + ks + fk];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bfg[j] = *(const bf16x8*)&sB[(wn + j * 16 + fr) * kLd + ks + fk];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfg[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    // accumulator (i, j)[r] is C[tm + wm + 16i + 4(lane/16) + r][tn + wn + 16j + lane%16]
-    if constexpr (EPI == EPI_PART) {
-        float* out = ep.part + ((size_t)blockIdx.z * gridDim.x * kBM) * ep.ldo;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int m0 = tm + wm + i * 16 + (lane >> 4) * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int n = tn + wn + j * 16 + fr;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) out[(size_t)(m0 + r) * ep.ldo + n] = acc[i][j][r];
-            }
-        }
-    } else if constexpr (EPI == EPI_FWD) {
-        // Z = acc + b, then H = silu(Z), each staged through LDS for row and column stores
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float b = ep.bias[tn + wn + j * 16 + fr];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    T[(wm + i * 16 + (lane >> 4) * 4 + r) * kTp + wn + j * 16 + fr] = (bf16)(acc[i][j][r] + b);
-        }
-        __syncthreads();
-        tile_store_rows(T, ep.z, ep.ldo, tm, tn);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float b = ep.bias[tn + wn + j * 16 + fr];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float z = acc[i][j][r] + b;
-                    T[(wm + i * 16 + (lane >> 4) * 4 + r) * kTp + wn + j * 16 + fr] = (bf16)(z * sigm(z));
-                }
-        }
-        __syncthreads();
-        tile_store_rows(T, ep.h, ep.ldo, tm, tn);
-        tile_store_cols(T, ep.ht, ep.ldt, tm, tn);
-    } else {
-        // dZ = dH * silu'(Z_prev): Z_prev tile into LDS (row loads), combined in place
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int id = threadIdx.x + 256 * it;
-            const int row = id >> 4, c8 = (id & 15) * 8;
-            *(uint4*)&T[row * kTp + c8] = *(const uint4*)&ep.zprev[(size_t)(tm + row) * ep.ldo + tn + c8];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    bf16& e = T[(wm + i * 16 + (lane >> 4) * 4 + r) * kTp + wn + j * 16 + fr];
-                    e = (bf16)(acc[i][j][r] * silu_grad((float)e));
-                }
-        __syncthreads();
-        tile_store_rows(T, ep.dz, ep.ldo, tm, tn);
-        tile_store_cols(T, ep.dzt, ep.ldt, tm, tn);
-    }
-}
-
-// ---- output layer --------------------------------------------------------------------
-// y[m] = H4[m] . w + b for rows m < mpad; one wave per row.
-__global__ void __launch_bounds__(256) k_head_fwd(int mpad, const bf16* __restrict__ H, const float* __restrict__ w,
-                                                  const float* __restrict__ b, float* __restrict__ y) {
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (m >= mpad) return;
-    const bf16* row = H + (size_t)m * kH + lane * 4;
-    float s = 0.0f;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) s = fmaf((float)row[c], w[lane * 4 + c], s);
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) y[m] = s + b[0];
-}
-
-// ---- inference in one pass -------------------------------------------------------------
-// Each block takes kPM rows through the embedding, the kL hidden layers and the output layer
-// with the rows' activations in one LDS tile (kPM x kH bf16, row stride kPLd): a layer's
-// products are accumulated in registers, the block synchronises, and the epilogue writes the
-// layer's output over its input.  The weights are MFMA operands read straight from the bf16
-// [out][in] copies (L2-resident).  Fragment mapping, k order (32 at a time), epilogue rounding
-// and the output layer's reduction are those of k_embed, k_gemm_nt<EPI_FWD> and k_head_fwd,
-// so y is bitwise the forward pass's; no per-row buffers, so any row count.
-constexpr int kPM = 64;        // rows per block
-constexpr int kPLd = kH + 8;   // LDS row stride (bf16): 16-byte aligned rows
-__global__ void __launch_bounds__(256) k_mlp_infer(int n, int nsets, const float* __restrict__ par,
-                                                   const int32_t* __restrict__ set, const float* __restrict__ q,
-                                                   const Features ft, const bf16* __restrict__ wb,
-                                                   const float* __restrict__ p, float* __restrict__ y) {
+// 4 waves per SIMD in both forms.  Training keeps Z in registers (64 of them with 8 waves), and
+// with two waves per SIMD its phases between barriers did not hide each other.
+template <bool TRAIN, int NW>
+__global__ void __launch_bounds__(64 * NW, 4) k_mlp(int n, int nsets, const float* __restrict__ par,
+                                             const int32_t* __restrict__ set, const float* __restrict__ q,
+                                             const Features ft, const bf16* __restrict__ wb,
+                                             const float* __restrict__ p, float* __restrict__ y, const TrainArgs tr) {
     __shared__ __attribute__((aligned(16))) bf16 act[kPM * kPLd];
+    __shared__ float s_y[kPM];
+    __shared__ __attribute__((aligned(16))) float s_sum[TRAIN ? NW / 2 : 1][kH];  // column sums of the row groups
     const int r0 = blockIdx.x * kPM;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    {
-        // embedding, four threads per row (k_embed's values, written to LDS one by one)
-        const int row = t >> 2, h = t & 3;
-        const int i = r0 + row;
-        bf16* dst = act + row * kPLd;
-        float v[kNP];
-#pragma unroll
-        for (int k = 0; k < kNP; ++k) v[k] = 0.0f;
-        const bool live = i < n;
-        float qx = 0.0f, qy = 0.0f;
-        if (live) {
-            const float* pp = par + (size_t)min(max(set[i], 0), nsets - 1) * kNP;  // clamped like k_embed
-#pragma unroll
-            for (int k = 0; k < kNP; ++k) v[k] = pp[k];
-            qx = q[2 * (size_t)i];
-            qy = q[2 * (size_t)i + 1];
-        }
-        const float qa = sqrtf(qx * qx + qy * qy);
-        if (h == 0)
-#pragma unroll
-            for (int k = 0; k < kNP; ++k) dst[k] = (bf16)v[k];
-#pragma unroll
-        for (int f0 = 0; f0 < kNF / 4; ++f0) {
-            const int f = h * (kNF / 4) + f0;
-            float sn = 0.0f, cs = 0.0f;
-            if (live) {
-                const int j = ft.pidx[f];
-                float pv = 1.0f;
-#pragma unroll
-                for (int k = 0; k < kNP; ++k) pv = (k == j) ? ft.off[k] + ft.sc[k] * v[k] : pv;
-                sincosf(6.283185307f * (ft.f[f][0] * qx + ft.f[f][1] * qy) + ft.f[f][2] * qa * pv, &sn, &cs);
-            }
-            dst[kNP + f] = (bf16)sn;
-            dst[kNP + kNF + f] = (bf16)cs;
-        }
-        for (int k = kUsed + h; k < kIn; k += 4) dst[k] = (bf16)0.0f;
-    }
+    constexpr int NI = 16 / NW;  // 16-feature tiles per wave
+    const int wn = wave * 16 * NI;
+    constexpr int64_t kW1 = (int64_t)kH * kIn, kWl = (int64_t)kH * kH;
+    bf16x4 z[TRAIN ? kL : 1][NI][4];  // pre-activations, kept for the backward pass
+    embed_rows<NW>(r0, n, nsets, par, set, q, ft, act);
     __syncthreads();
-    const int fr = lane & 15, fk = (lane >> 4) * 8;
-    const int wn = wave * 64;  // this wave's 64 output columns
+    if constexpr (TRAIN) store_columns<NW, false>(act, tr.xt + (size_t)r0 * kIn, kIn, nullptr);
+#pragma unroll
     for (int l = 0; l < kL; ++l) {
-        const int K = in_of(l);
-        const bf16* W = wb + (l == 0 ? 0 : (int64_t)kH * kIn + (int64_t)(l - 1) * kH * kH);
-        f32x4 acc[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        for (int ks = 0; ks < K; ks += 32) {
-            bf16x8 af[4], bfg[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bfg[j] = *(const bf16x8*)&W[(size_t)(wn + j * 16 + fr) * K + ks + fk];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) af[i] = *(const bf16x8*)&act[(i * 16 + fr) * kPLd + ks + fk];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfg[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();  // every wave has read the layer's input
+        f32x4 acc[NI][4];
         const float* b = p + b_off(l);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float bj = b[wn + j * 16 + fr];
+        for (int i = 0; i < NI; ++i) {
+            const f32x4 bi = {b[acc_feature(wn, i)], b[acc_feature(wn, i) + 1], b[acc_feature(wn, i) + 2],
+                              b[acc_feature(wn, i) + 3]};
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int j = 0; j < 4; ++j) acc[i][j] = bi;
+        }
+        if (l == 0) layer_product<kIn, NI, !TRAIN>(wb, act, wn, acc);
+        else layer_product<kH, NI, !TRAIN>(wb + kW1 + (l - 1) * kWl, act, wn, acc);
+        __syncthreads();  // every wave has read the layer's input
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                bf16x4 h;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float z = acc[i][j][r] + bj;
-                    act[(i * 16 + (lane >> 4) * 4 + r) * kPLd + wn + j * 16 + fr] = (bf16)(z * sigm(z));
+                    const float zz = acc[i][j][r];
+                    h[r] = (bf16)(zz * sigm(zz));
+                    if constexpr (TRAIN) z[l][i][j][r] = (bf16)zz;
                 }
-        }
+                *(bf16x4*)&act[acc_row(j) * kPLd + acc_feature(wn, i)] = h;
+            }
         __syncthreads();
+        if constexpr (TRAIN)
+            if (l < kL - 1) store_columns<NW, false>(act, tr.ht[l] + (size_t)r0 * kH, kH, nullptr);
     }
+    // output layer: one wave per row
     const float* w = p + kOutW;
-    for (int rr = wave; rr < kPM; rr += 4) {
+    for (int rr = wave; rr < kPM; rr += NW) {
         const bf16* row = act + rr * kPLd + lane * 4;
         float sum = 0.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) sum = fmaf((float)row[c], w[lane * 4 + c], sum);
         for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-        if (lane == 0 && r0 + rr < n) y[r0 + rr] = sum + p[kOutB];
-    }
-}
-
-// Loss 1/n sum (y - t)^2 and the output layer's backward for a block of kHeadRows rows:
-// dy = 2 (y - t) / n (0 for rows >= n) into dy_out, dZ4[m][c] = dy * w[c] * silu'(Z4[m][c])
-// written in both layouts, and per-block partials of db = sum dy and of the loss.
-__global__ void __launch_bounds__(256) k_head_bwd(int n, int mpad, const float* __restrict__ y,
-                                                  const float* __restrict__ tgt, const bf16* __restrict__ Z,
-                                                  const float* __restrict__ w, float* __restrict__ dy_out,
-                                                  bf16* __restrict__ dZ, bf16* __restrict__ dZT,
-                                                  float* __restrict__ part_b) {
-    __shared__ bf16 tile[kHeadRows][kH + 8];
-    __shared__ float s_dy[kHeadRows];
-    const int m0 = blockIdx.x * kHeadRows, t = threadIdx.x;
-    if (t < kHeadRows) {
-        const int m = m0 + t;
-        const float dy = (m < n) ? 2.0f * (y[m] - tgt[m]) / (float)n : 0.0f;
-        s_dy[t] = dy;
-        dy_out[m] = dy;
-    }
-    __syncthreads();
-    // thread t owns column c = t
-    const int c = t;
-    const float wc = w[c];
-    for (int r = 0; r < kHeadRows; ++r) {
-        const size_t o = (size_t)(m0 + r) * kH + c;
-        const bf16 dz = (bf16)(s_dy[r] * wc * silu_grad((float)Z[o]));
-        tile[r][c] = dz;
-        dZ[o] = dz;
-    }
-    // column c of the tile is 64 consecutive rows of dZ^T
-    bf16* dst = dZT + (size_t)c * mpad + m0;
-#pragma unroll
-    for (int r = 0; r < kHeadRows; r += 8) {
-        bf16x8 pk;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pk[j] = tile[r + j][c];
-        *(bf16x8*)(dst + r) = pk;
-    }
-    if (t == 0) {
-        float db = 0.0f, loss = 0.0f;
-        for (int r = 0; r < kHeadRows; ++r) {
-            db += s_dy[r];
-            const int m = m0 + r;
-            if (m < n) loss += (y[m] - tgt[m]) * (y[m] - tgt[m]);
-        }
-        part_b[2 * blockIdx.x] = db;
-        part_b[2 * blockIdx.x + 1] = loss;
-    }
-}
-
-__device__ __forceinline__ float block_sum(float v, float* red) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    const float s = red[0] + red[1] + red[2] + red[3];
-    __syncthreads();
-    return s;
-}
-
-// Row reductions over the batch for rows of a [rows][mpad] bf16 matrix, in segments of
-// kSeg columns: part[r * S + s] = sum over the segment of A[r][m] * (w ? w[m] : 1).
-// Grid (rows, S = ceil(mpad / kSeg)); each thread takes one 8-column chunk.
-constexpr int kSeg = 256 * 8;
-__global__ void __launch_bounds__(256) k_rowdot(int mpad, const bf16* __restrict__ A, const float* __restrict__ w,
-                                                float* __restrict__ part) {
-    __shared__ float red[4];
-    const int r = blockIdx.x, sg = blockIdx.y;
-    const int m = sg * kSeg + threadIdx.x * 8;
-    float acc = 0.0f;
-    if (m < mpad) {  // mpad is a multiple of 128: chunks lie wholly inside or outside
-        const bf16x8 v = *(const bf16x8*)(A + (size_t)r * mpad + m);
-        if (w) {
-            const float4 w0 = *(const float4*)(w + m), w1 = *(const float4*)(w + m + 4);
-            acc = (float)v[0] * w0.x + (float)v[1] * w0.y + (float)v[2] * w0.z + (float)v[3] * w0.w +
-                  (float)v[4] * w1.x + (float)v[5] * w1.y + (float)v[6] * w1.z + (float)v[7] * w1.w;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc += (float)v[j];
+        if (lane == 0) {
+            sum += p[kOutB];
+            if constexpr (TRAIN) s_y[rr] = sum;
+            else if (r0 + rr < n) y[r0 + rr] = sum;
         }
     }
-    const float s = block_sum(acc, red);
-    if (threadIdx.x == 0) part[(size_t)r * gridDim.y + sg] = s;
-}
-// out[r] = sum over s < S of part[r * S + s] (fixed order)
-__global__ void k_rowdot_finish(int rows, int S, const float* __restrict__ part, float* __restrict__ out) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
-    float s = 0.0f;
-    for (int k = 0; k < S; ++k) s += part[(size_t)r * S + k];
-    out[r] = s;
-}
-
-// Sums of the output layer's block partials: g_b = sum db, loss_sum = sum loss (one block).
-__global__ void __launch_bounds__(256) k_head_finish(int nb, const float* __restrict__ part_b, float* __restrict__ g_b,
-                                                     float* __restrict__ loss_sum) {
-    __shared__ float red[4];
-    float db = 0.0f, ls = 0.0f;
-    for (int k = threadIdx.x; k < nb; k += 256) {
-        db += part_b[2 * k];
-        ls += part_b[2 * k + 1];
-    }
-    db = block_sum(db, red);
-    ls = block_sum(ls, red);
-    if (threadIdx.x == 0) {
-        *g_b = db;
-        *loss_sum = ls;
-    }
-}
-
-// g[c] = sum over s < ns of part[s*ld + c] for the weight-gradient splits, 4 columns per
-// thread (fixed order: deterministic).
-__global__ void __launch_bounds__(256) k_sum_parts(int n4, int ns, int ld4, const float4* __restrict__ part,
-                                                   float4* __restrict__ g) {
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n4) return;
-    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (TRAIN) {
+        // loss 1/n sum (y - t)^2: dy = 2 (y - t) / n, 0 for rows >= n
+        __syncthreads();
+        float* part = tr.part + (size_t)blockIdx.x * kPartB;
+        auto sum_groups = [&](float* out) {  // a barrier after the groups' sums
+            if (t < kH) {
+                float v = s_sum[0][t];
+#pragma unroll
+                for (int g = 1; g < NW / 2; ++g) v += s_sum[g][t];
+                out[t] = v;
+            }
+        };
+        if (t < kPM) {
+            const float e = r0 + t < n ? s_y[t] - tr.tgt[r0 + t] : 0.0f;
+            const float dy = 2.0f * e / (float)n;
+            s_y[t] = dy;
+            float db = dy, ls = e * e;
+            for (int o = 32; o > 0; o >>= 1) {
+                db += __shfl_xor(db, o, 64);
+                ls += __shfl_xor(ls, o, 64);
+            }
+            if (t == 0) {
+                part[(kL + 1) * kH] = db;
+                part[(kL + 1) * kH + 1] = ls;
+            }
+        }
+        __syncthreads();
+        {
+            // output weights: dw[c] = sum over the rows of dy H_kL[row][c], rows and features
+            // split as in store_columns
+            constexpr int R = 2 * kPM / NW;
+            const int c = (t & 127) * 2, h = (t >> 7) * R;
+            float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll 8
-    for (int k = 0; k < ns; ++k) {
-        const float4 v = part[(size_t)k * ld4 + c];
-        s.x += v.x;
-        s.y += v.y;
-        s.z += v.z;
-        s.w += v.w;
+            for (int r = 0; r < R; ++r) {
+                const uint32_t x = *(const uint32_t*)&act[(h + r) * kPLd + c];
+                s0 = fmaf(__uint_as_float(x << 16), s_y[h + r], s0);
+                s1 = fmaf(__uint_as_float(x & 0xffff0000u), s_y[h + r], s1);
+            }
+            *(float2*)&s_sum[t >> 7][c] = make_float2(s0, s1);
+        }
+        __syncthreads();  // the last activations are read
+        sum_groups(part + kL * kH);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float dy = s_y[acc_row(j)];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                bf16x4 dz;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    dz[r] = (bf16)(dy * w[acc_feature(wn, i) + r] * silu_grad((float)z[kL - 1][i][j][r]));
+                *(bf16x4*)&act[acc_row(j) * kPLd + acc_feature(wn, i)] = dz;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int l = kL - 1; l >= 0; --l) {
+            // dZ_l^T and the bias gradient's partials
+            store_columns<NW, true>(act, tr.dzt[l] + (size_t)r0 * kH, kH, s_sum[0]);
+            if (l == 0) {
+                __syncthreads();
+                sum_groups(part);
+                break;
+            }
+            // dH_{l-1} = dZ_l . W_l, dZ_{l-1} = dH_{l-1} silu'(Z_{l-1})
+            f32x4 acc[NI][4];
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            layer_product<kH, NI, false>(tr.wtb + kW1 + (l - 1) * kWl, act, wn, acc);
+            __syncthreads();
+            sum_groups(part + l * kH);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < NI; ++i) {
+                    bf16x4 dz;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        dz[r] = (bf16)(acc[i][j][r] * silu_grad((float)z[l - 1][i][j][r]));
+                    *(bf16x4*)&act[acc_row(j) * kPLd + acc_feature(wn, i)] = dz;
+                }
+            __syncthreads();
+        }
     }
-    g[c] = s;
+}
+
+// ---- weight gradients --------------------------------------------------------------------
+// part_l[split][out][in] = sum over the split's rows of dZ_l[m][out] H_{l-1}[m][in]: block x
+// takes layer x whole (256 outputs x its inputs), block y the split, so every operand byte is
+// read by one block only.  8 waves, 4 x 2, each 64 outputs x half of the inputs; the operands lie
+// in fragment order and go straight to registers, the next k step's while this one is
+// multiplied.  Bound: the operands' bytes, 235 MB at 65,536 rows (50 us at 4.8 TB/s).  As 128 x 128
+// tiles through LDS, per layer, each byte was read by two blocks, seldom on one XCD.
+struct WgradArgs {
+    const bf16* dzt[kL];
+    const bf16* ht[kL];  // layer inputs: X^T, H_0^T, ...
+    float* part[kL];     // [splits][kH][in]
+    int nb, kchunk;      // row blocks of kPM, row blocks per split
+};
+template <int K>
+__device__ __forceinline__ void wgrad_layer(const bf16* __restrict__ A, const bf16* __restrict__ B,
+                                            float* __restrict__ out, int k0, int k1) {
+    constexpr int NJ = K / 32;  // 16-column tiles per wave
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave & 3) * 64, wn = (wave >> 2) * (K / 2);
+    const bf16* ap = A + (size_t)(wm / 16) * 512 + lane * 8;
+    const bf16* bp = B + (size_t)(wn / 16) * 512 + lane * 8;
+    // a block's kPM rows are two k steps of kH / 16 and K / 16 fragments each
+    f32x4 acc[4][NJ];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 a[4], b[NJ], an[4], bn[NJ];
+    const int s0 = 2 * k0, s1 = 2 * k1;
+    auto fetch = [&](int st, bf16x8* fa, bf16x8* fb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) fa[i] = *(const bf16x8*)(ap + ((size_t)st * (kH / 16) + i) * 512);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) fb[j] = *(const bf16x8*)(bp + ((size_t)st * (K / 16) + j) * 512);
+    };
+    auto multiply = [&](const bf16x8* fa, const bf16x8* fb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    };
+    fetch(s0, a, b);
+#pragma unroll 1
+    for (int st = s0; st < s1; st += 2) {  // an even number of steps
+        fetch(st + 1, an, bn);
+        multiply(a, b);
+        fetch(min(st + 2, s1 - 2), a, b);
+        multiply(an, bn);
+    }
+    // accumulator (i, j)[r] is C[wm + 16i + 4(lane/16) + r][wn + 16j + lane%16]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m0 = wm + i * 16 + (lane >> 4) * 4;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int c = wn + j * 16 + (lane & 15);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[(size_t)(m0 + r) * K + c] = acc[i][j][r];
+        }
+    }
+}
+__global__ void __launch_bounds__(512, 2) k_wgrad(const WgradArgs g) {
+    const int l = blockIdx.x;
+    const int k0 = blockIdx.y * g.kchunk, k1 = min(g.nb, k0 + g.kchunk);
+    if (k0 >= k1) return;
+    if (l == 0) wgrad_layer<kIn>(g.dzt[0], g.ht[0], g.part[0] + (size_t)blockIdx.y * kH * kIn, k0, k1);
+    else wgrad_layer<kH>(g.dzt[l], g.ht[l], g.part[l] + (size_t)blockIdx.y * kH * kH, k0, k1);
+}
+
+// The packed gradient from the partials, each sum in a fixed order: blocks below kFinW take 1024
+// weights each (four per thread, summed over the splits), the others 16 of the kPartB sums over
+// the nr row blocks (16 threads per value, then a tree).
+constexpr int kFinW = (int)((kH * kIn + (kL - 1) * (int64_t)kH * kH) / 1024);
+constexpr int kFinB = (kPartB + 15) / 16;
+struct FinishArgs {
+    const float* part[kL];
+    const float* pb;   // [nr][kPartB]
+    float* g;          // packed gradient
+    float* loss;       // sum of the squared errors
+    int ns, nr;
+};
+__global__ void __launch_bounds__(256) k_finish(const FinishArgs a) {
+    const int t = threadIdx.x;
+    if ((int)blockIdx.x < kFinW) {
+        int c = blockIdx.x * 1024 + t * 4, l = 0;
+        if (c >= kH * kIn) {
+            c -= kH * kIn;
+            l = 1 + c / (kH * kH);
+            c %= kH * kH;
+        }
+        const int sz = kH * in_of(l);
+        float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 8
+        for (int k = 0; k < a.ns; ++k) {
+            const float4 v = *(const float4*)&a.part[l][(size_t)k * sz + c];
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
+        }
+        float* o = a.g + w_off(l) + c;
+        o[0] = s.x;
+        o[1] = s.y;
+        o[2] = s.z;
+        o[3] = s.w;
+        return;
+    }
+    __shared__ float red[16][17];
+    const int vi = t & 15, sg = t >> 4;
+    const int v = ((int)blockIdx.x - kFinW) * 16 + vi;
+    float s = 0.0f;
+    if (v < kPartB)
+#pragma unroll 8
+        for (int k = sg; k < a.nr; k += 16) s += a.pb[(size_t)k * kPartB + v];
+    red[sg][vi] = s;
+    __syncthreads();
+    for (int h = 8; h > 0; h >>= 1) {
+        if (sg < h) red[sg][vi] += red[sg + h][vi];
+        __syncthreads();
+    }
+    if (sg == 0 && v < kPartB) {
+        const float r = red[0][vi];
+        if (v < kL * kH) a.g[b_off(v / kH) + v % kH] = r;
+        else if (v < (kL + 1) * kH) a.g[kOutW + v - kL * kH] = r;
+        else if (v == (kL + 1) * kH) a.g[kOutB] = r;
+        else *a.loss = r;
+    }
 }
 
 // Adam on the FP32 master parameters, then the bf16 copies of the hidden weights in both
-// orientations (W [out][in] and W^T [in][out]).
+// orientations (W and W^T), in the order in which k_mlp's waves read them.
 __global__ void __launch_bounds__(256) k_adam(int64_t np, float* __restrict__ p, const float* __restrict__ g,
                                               float* __restrict__ m1, float* __restrict__ m2, float lr, float b1,
                                               float b2, float eps, float c1, float c2) {
@@ -529,8 +557,8 @@ __global__ void __launch_bounds__(256) k_cast_weights(const float* __restrict__ 
             const int o = (int)(i / in_of(l)), k = (int)(i % in_of(l));
             const bf16 v = (bf16)p[w_off(l) + i];
             const int64_t base = l == 0 ? 0 : (int64_t)kH * kIn + (int64_t)(l - 1) * kH * kH;
-            wb[base + i] = v;
-            wtb[base + (int64_t)k * kH + o] = v;
+            wb[base + frag_index(o, k, kH)] = v;
+            wtb[base + frag_index(k, o, in_of(l))] = v;
             return;
         }
         i -= cnt;
@@ -555,11 +583,9 @@ struct csx_mlp {
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
     bf16 *wb = nullptr, *wtb = nullptr;  // hidden weights, [out][in] and [in][out]
     int64_t adam_t = 0;
-    // per-row buffers
-    bf16 *X = nullptr, *XT = nullptr;
-    bf16 *Z[kL] = {}, *H[kL] = {}, *HT[kL] = {};
-    bf16 *dZ[2] = {}, *dZT[2] = {};
-    float *y = nullptr, *dy = nullptr, *part = nullptr, *rpart = nullptr, *hpart_b = nullptr, *loss = nullptr;
+    // training buffers: the layers' inputs and dZ, transposed; partial sums
+    bf16 *XT = nullptr, *HT[kL - 1] = {}, *dZT[kL] = {};
+    float *part = nullptr, *pb = nullptr, *loss = nullptr;
     int splits = 0;
 };
 
@@ -574,13 +600,6 @@ int fail(csx_mlp* m, int code, const std::string& msg) {
         hipError_t e_ = (call);                                                              \
         if (e_ != hipSuccess) return fail(m, CSX_E_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-const bf16* wb_layer(const csx_mlp* m, int l) {
-    return m->wb + (l == 0 ? 0 : (int64_t)kH * kIn + (int64_t)(l - 1) * kH * kH);
-}
-const bf16* wtb_layer(const csx_mlp* m, int l) {
-    return m->wtb + (l == 0 ? 0 : (int64_t)kH * kIn + (int64_t)(l - 1) * kH * kH);
-}
 
 // splitmix64 -> uniform doubles, Box-Muller normals (host-side initialisation only)
 struct Rng {
@@ -607,28 +626,9 @@ int check_rows(csx_mlp* m, int n, int nsets) {
     return CSX_OK;
 }
 
-// Forward pass over n rows (padded to a multiple of 128) into m->y.
-int forward(csx_mlp* m, int n, int nsets, const float* d_par, const int32_t* d_set, const float* d_q) {
-    const int mpad = (n + kBM - 1) / kBM * kBM;
-    hipLaunchKernelGGL(k_embed, dim3((mpad + 255) / 256), dim3(256), 0, m->stream, n, mpad, nsets, d_par, d_set, d_q,
-                       m->feat, m->X, m->XT);
-    MCHK(m, hipGetLastError());
-    for (int l = 0; l < kL; ++l) {
-        EpiArgs ep{};
-        ep.bias = m->p + b_off(l);
-        ep.z = m->Z[l];
-        ep.h = m->H[l];
-        ep.ht = m->HT[l];
-        ep.ldo = kH;
-        ep.ldt = mpad;
-        const bf16* A = l == 0 ? m->X : m->H[l - 1];
-        const int K = in_of(l);
-        hipLaunchKernelGGL(k_gemm_nt<EPI_FWD>, dim3(mpad / kBM, kH / kBN, 1), dim3(256), 0, m->stream, A, K,
-                           wb_layer(m, l), K, K, K, ep);
-        MCHK(m, hipGetLastError());
-    }
-    hipLaunchKernelGGL(k_head_fwd, dim3(mpad / 4), dim3(256), 0, m->stream, mpad, m->H[kL - 1], m->p + kOutW,
-                       m->p + kOutB, m->y);
+int infer(csx_mlp* m, int n, int nsets, const float* d_par, const int32_t* d_set, const float* d_q, float* d_y) {
+    hipLaunchKernelGGL((k_mlp<false, kInferWaves>), dim3((unsigned)((n + kPM - 1) / kPM)), dim3(64 * kInferWaves), 0, m->stream, n, nsets, d_par,
+                       d_set, d_q, m->feat, m->wb, m->p, d_y, TrainArgs{});
     MCHK(m, hipGetLastError());
     return CSX_OK;
 }
@@ -647,7 +647,8 @@ int csx_mlp_create(int device, int max_batch, uint64_t seed, csx_mlp** out) {
     m->device = device;
     m->max_batch = (max_batch + kBM - 1) / kBM * kBM;
     const size_t M = (size_t)m->max_batch;
-    // weight-gradient splits over the rows: enough blocks to fill the chip, >= 512 rows each
+    // weight-gradient splits over the rows, >= 512 rows each: 64 give one block per CU (4 layers);
+    // every split writes and reads 0.9 MB of partials
     m->splits = (int)std::max<size_t>(1, std::min<size_t>(64, M / 512));
     auto alloc = [&](void** p, size_t bytes) { return hipMalloc(p, bytes) == hipSuccess; };
     bool ok = hipStreamCreate(&m->stream) == hipSuccess;
@@ -656,14 +657,10 @@ int csx_mlp_create(int device, int max_batch, uint64_t seed, csx_mlp** out) {
     ok = ok && alloc((void**)&m->p, kNParams * 4) && alloc((void**)&m->g, kNParams * 4) &&
          alloc((void**)&m->m1, kNParams * 4) && alloc((void**)&m->m2, kNParams * 4) &&
          alloc((void**)&m->wb, nw * 2) && alloc((void**)&m->wtb, nw * 2) &&
-         alloc((void**)&m->X, M * kIn * 2) && alloc((void**)&m->XT, M * kIn * 2) && alloc((void**)&m->y, M * 4) &&
-         alloc((void**)&m->dy, M * 4) && alloc((void**)&m->part, (size_t)m->splits * kH * kH * 4) &&
-         alloc((void**)&m->rpart, (size_t)kH * ((M + kSeg - 1) / kSeg) * 4) &&
-         alloc((void**)&m->hpart_b, (M / kHeadRows) * 2 * 4) && alloc((void**)&m->loss, 4);
-    for (int l = 0; l < kL && ok; ++l)
-        ok = alloc((void**)&m->Z[l], M * kH * 2) && alloc((void**)&m->H[l], M * kH * 2) &&
-             alloc((void**)&m->HT[l], M * kH * 2);
-    for (int k = 0; k < 2 && ok; ++k) ok = alloc((void**)&m->dZ[k], M * kH * 2) && alloc((void**)&m->dZT[k], M * kH * 2);
+         alloc((void**)&m->XT, M * kIn * 2) && alloc((void**)&m->part, (size_t)m->splits * nw * 4) &&
+         alloc((void**)&m->pb, (M / kPM) * kPartB * 4) && alloc((void**)&m->loss, 4);
+    for (int l = 0; l < kL - 1 && ok; ++l) ok = alloc((void**)&m->HT[l], M * kH * 2);
+    for (int l = 0; l < kL && ok; ++l) ok = alloc((void**)&m->dZT[l], M * kH * 2);
     if (!ok) {
         csx_mlp_destroy(m);
         return CSX_E_NOMEM;
@@ -708,15 +705,12 @@ void csx_mlp_destroy(csx_mlp* m) {
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     for (void* q : {(void*)m->p, (void*)m->g, (void*)m->m1, (void*)m->m2, (void*)m->wb, (void*)m->wtb,
-                    (void*)m->X, (void*)m->XT, (void*)m->y, (void*)m->dy, (void*)m->part, (void*)m->rpart,
-                    (void*)m->hpart_b, (void*)m->loss})
+                    (void*)m->XT, (void*)m->part, (void*)m->pb, (void*)m->loss})
         if (q) (void)hipFree(q);
-    for (int l = 0; l < kL; ++l)
-        for (void* q : {(void*)m->Z[l], (void*)m->H[l], (void*)m->HT[l]})
-            if (q) (void)hipFree(q);
-    for (int k = 0; k < 2; ++k)
-        for (void* q : {(void*)m->dZ[k], (void*)m->dZT[k]})
-            if (q) (void)hipFree(q);
+    for (bf16* q : m->HT)
+        if (q) (void)hipFree(q);
+    for (bf16* q : m->dZT)
+        if (q) (void)hipFree(q);
     if (m->own_stream && m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -800,20 +794,14 @@ int csx_mlp_forward(csx_mlp* m, int n, int nsets, const float* d_par, const int3
     int rc = check_rows(m, n, nsets);
     if (rc) return rc;
     MCHK(m, hipSetDevice(m->device));
-    rc = forward(m, n, nsets, d_par, d_set, d_q);
-    if (rc) return rc;
-    MCHK(m, hipMemcpyAsync(d_y, m->y, (size_t)n * 4, hipMemcpyDeviceToDevice, m->stream));
-    return CSX_OK;
+    return infer(m, n, nsets, d_par, d_set, d_q, d_y);
 }
 
 int csx_mlp_predict(csx_mlp* m, int n, int nsets, const float* d_par, const int32_t* d_set, const float* d_q,
                     float* d_y) {
     if (!m || !d_par || !d_set || !d_q || !d_y || n < 1 || nsets < 1) return CSX_E_ARG;
     MCHK(m, hipSetDevice(m->device));
-    hipLaunchKernelGGL(k_mlp_infer, dim3((unsigned)((n + kPM - 1) / kPM)), dim3(256), 0, m->stream, n, nsets, d_par,
-                       d_set, d_q, m->feat, m->wb, m->p, d_y);
-    MCHK(m, hipGetLastError());
-    return CSX_OK;
+    return infer(m, n, nsets, d_par, d_set, d_q, d_y);
 }
 
 int csx_mlp_gradient(csx_mlp* m, int n, int nsets, const float* d_par, const int32_t* d_set, const float* d_q,
@@ -822,53 +810,38 @@ int csx_mlp_gradient(csx_mlp* m, int n, int nsets, const float* d_par, const int
     int rc = check_rows(m, n, nsets);
     if (rc) return rc;
     MCHK(m, hipSetDevice(m->device));
-    rc = forward(m, n, nsets, d_par, d_set, d_q);
-    if (rc) return rc;
-    const int mpad = (n + kBM - 1) / kBM * kBM;
-    const int nhb = mpad / kHeadRows;
-    const int nseg = (mpad + kSeg - 1) / kSeg;
-    // output layer: dy, dZ of the last hidden layer, db and the loss; dw = H4^T . dy
-    hipLaunchKernelGGL(k_head_bwd, dim3(nhb), dim3(256), 0, m->stream, n, mpad, m->y, d_t, m->Z[kL - 1],
-                       m->p + kOutW, m->dy, m->dZ[0], m->dZT[0], m->hpart_b);
-    MCHK(m, hipGetLastError());
-    hipLaunchKernelGGL(k_head_finish, dim3(1), dim3(256), 0, m->stream, nhb, m->hpart_b, m->g + kOutB, m->loss);
-    hipLaunchKernelGGL(k_rowdot, dim3(kH, nseg), dim3(256), 0, m->stream, mpad, m->HT[kL - 1], m->dy, m->rpart);
-    hipLaunchKernelGGL(k_rowdot_finish, dim3(1), dim3(kH), 0, m->stream, kH, nseg, m->rpart, m->g + kOutW);
-    MCHK(m, hipGetLastError());
-    // hidden layers, top down; dZ of layer l is in buffer cur
-    int cur = 0;
-    for (int l = kL - 1; l >= 0; --l) {
-        const int K = in_of(l);
-        // weight gradient dW_l [kH][K] = dZ_l^T . H_{l-1}, split over the rows
-        const int kchunk = ((mpad / m->splits + kBK - 1) / kBK) * kBK;
-        const int ns = (mpad + kchunk - 1) / kchunk;
-        EpiArgs pe{};
-        pe.part = m->part;
-        pe.ldo = K;
-        const bf16* BT = l == 0 ? m->XT : m->HT[l - 1];
-        hipLaunchKernelGGL(k_gemm_nt<EPI_PART>, dim3(kH / kBM, K / kBN, ns), dim3(256), 0, m->stream, m->dZT[cur], mpad,
-                           BT, mpad, mpad, kchunk, pe);
-        MCHK(m, hipGetLastError());
-        const int n4 = kH * K / 4;
-        hipLaunchKernelGGL(k_sum_parts, dim3((n4 + 255) / 256), dim3(256), 0, m->stream, n4, ns, n4,
-                           (const float4*)m->part, (float4*)(m->g + w_off(l)));
-        // bias gradient: row sums of dZ^T
-        hipLaunchKernelGGL(k_rowdot, dim3(kH, nseg), dim3(256), 0, m->stream, mpad, m->dZT[cur], nullptr, m->rpart);
-        hipLaunchKernelGGL(k_rowdot_finish, dim3(1), dim3(kH), 0, m->stream, kH, nseg, m->rpart, m->g + b_off(l));
-        MCHK(m, hipGetLastError());
-        if (l == 0) break;
-        // dH_{l-1} = dZ_l . W_l, then dZ_{l-1} = dH_{l-1} * silu'(Z_{l-1})
-        EpiArgs be{};
-        be.zprev = m->Z[l - 1];
-        be.dz = m->dZ[cur ^ 1];
-        be.dzt = m->dZT[cur ^ 1];
-        be.ldo = kH;
-        be.ldt = mpad;
-        hipLaunchKernelGGL(k_gemm_nt<EPI_BWD>, dim3(mpad / kBM, kH / kBN, 1), dim3(256), 0, m->stream, m->dZ[cur], kH,
-                           wtb_layer(m, l), kH, kH, kH, be);
-        MCHK(m, hipGetLastError());
-        cur ^= 1;
+    const int nb = (n + kPM - 1) / kPM;
+    const int64_t w1 = (int64_t)kH * kIn, wl = (int64_t)kH * kH;
+    TrainArgs tr{};
+    WgradArgs wg{};
+    FinishArgs fa{};
+    tr.tgt = d_t;
+    tr.xt = m->XT;
+    tr.wtb = m->wtb;
+    tr.part = m->pb;
+    wg.nb = nb;
+    for (int l = 0; l < kL; ++l) {
+        if (l < kL - 1) tr.ht[l] = m->HT[l];
+        tr.dzt[l] = m->dZT[l];
+        wg.dzt[l] = m->dZT[l];
+        wg.ht[l] = l == 0 ? m->XT : m->HT[l - 1];
+        wg.part[l] = m->part + (l == 0 ? 0 : m->splits * (w1 + (l - 1) * wl));
+        fa.part[l] = wg.part[l];
     }
+    hipLaunchKernelGGL((k_mlp<true, kTrainWaves>), dim3(nb), dim3(64 * kTrainWaves), 0, m->stream, n, nsets, d_par, d_set, d_q, m->feat, m->wb, m->p,
+                       (float*)nullptr, tr);
+    MCHK(m, hipGetLastError());
+    wg.kchunk = (nb + m->splits - 1) / m->splits;
+    const int ns = (nb + wg.kchunk - 1) / wg.kchunk;
+    hipLaunchKernelGGL(k_wgrad, dim3(kL, ns), dim3(512), 0, m->stream, wg);
+    MCHK(m, hipGetLastError());
+    fa.pb = m->pb;
+    fa.g = m->g;
+    fa.loss = m->loss;
+    fa.ns = ns;
+    fa.nr = nb;
+    hipLaunchKernelGGL(k_finish, dim3(kFinW + kFinB), dim3(256), 0, m->stream, fa);
+    MCHK(m, hipGetLastError());
     if (h_loss) {
         float ls = 0.0f;
         MCHK(m, hipMemcpyAsync(&ls, m->loss, 4, hipMemcpyDeviceToHost, m->stream));

@@ -145,3 +145,20 @@ def test_training_is_deterministic_with_fresh_batches():
         net.synchronize()
         out.append(net.get_params())
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 513, 4160])
+def test_gradient_rows(n):
+    """Row counts around the 64-row blocks and the splits of the weight gradient: the gradient of
+    n rows against the oracle's, and rows beyond n leave no trace (a second call on other rows
+    first)."""
+    net = _net(max_batch=4200, seed=6, physics=True)
+    (_, _, _, _), (bp, bs, bq, bt) = _inputs(4200, seed=1)
+    net.gradient(bp, bs, bq, bt)
+    (par, sets, q, t), (dpar, dsets, dq, dt) = _inputs(n, seed=20 + n)
+    loss = net.gradient(dpar, dsets, dq, dt)
+    g = net.get_grads().astype(np.float64)
+    X = mo.features(par, sets, q, *net.get_features())
+    lb, gb = mo.loss_and_grad(net.get_params().astype(np.float64), X, t, bf16=True)
+    assert abs(loss - lb) <= 2e-2 * lb                           # bf16 activations: 8-bit mantissas
+    assert np.linalg.norm(g - gb) <= 2e-2 * np.linalg.norm(gb)   # as for the whole batch
