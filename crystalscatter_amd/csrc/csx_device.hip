@@ -1163,50 +1163,81 @@ __device__ double romb_delta_cyl(const DevSet& d, double qx, double qy, int i1) 
 // with (X, Y) = (qxs^2, qys^2), swapped for case 3.  The inner sum is evaluated by Horner in
 // the ratio of the smaller to the larger of X and Y (no power tables; the reference builds
 // X^m and Y^(n-m) as running products, so the two agree to rounding).
-__device__ double cyl_gauss_series(const DevSet& d, double qxs, double qys, int oc) {
+// Wave-cooperative (called by all 64 lanes; `want` per lane): the requesting lanes are taken one
+// at a time (of nparts waves with the same pixels, this one takes every nparts-th request), and
+// lane j forms the inner sum and powers of order n = j + 1 (then j + 65); the terms are added in
+// order.  One lane on its own walks up
+// to 120 x 120 / 2 dependent loads where the series does not converge: 0.2 ms, longer than the
+// rest of a 512^2 pattern.
+__device__ double cyl_gauss_series(const DevSet& d, double qxs, double qys, int oc, bool want, int part, int nparts) {
     const double* c1p = carr_of<0>(d);
     const double* c11 = d.carr11pm;  // [n][m], CSX_NIM2 columns
-    const double X = (oc == 3) ? qys * qys : qxs * qxs, Y = (oc == 3) ? qxs * qxs : qys * qys;
-    const bool xs = X <= Y;            // Horner variable r = small/large <= 1
-    const double big = xs ? Y : X, r = xs ? (Y > 0 ? X / Y : 0.0) : (X > 0 ? Y / X : 0.0);
-    double pql = 1.0, old = 0.0, bn = 1.0;
-#pragma unroll 1
-    for (int n = 1; n <= 120; ++n) {
-        bn *= big;
-        // sum_m c11[n-m][m] X^m Y^(n-m) = big^n * sum_k a_k r^k, with k = m (X small) or n-m
-        double h = xs ? c11[0 * CSX_NIM2 + n] : c11[n * CSX_NIM2 + 0];
-#pragma unroll 1
-        for (int k = n - 1; k >= 0; --k) {
-            const double a = xs ? c11[(n - k) * CSX_NIM2 + k] : c11[k * CSX_NIM2 + (n - k)];
-            h = h * r + a;
+    const int lane = (int)threadIdx.x & 63;
+    unsigned long long todo = __ballot(want);
+    double mine = 1.0;
+    for (int i = 0; todo; ++i) {
+        const int l = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        if (i % nparts != part) continue;
+        const double px = __shfl(qxs, l, 64), py = __shfl(qys, l, 64);
+        const double X = (oc == 3) ? py * py : px * px, Y = (oc == 3) ? px * px : py * py;
+        const bool xs = X <= Y;            // Horner variable r = small/large <= 1
+        const double big = xs ? Y : X, r = xs ? (Y > 0 ? X / Y : 0.0) : (X > 0 ? Y / X : 0.0);
+        double pql = 1.0, old = 0.0;
+        bool go = true;
+        for (int base = 0; go && base < 120; base += 64) {
+            const int n = min(base + 1 + lane, 120);
+            // sum_m c11[n-m][m] X^m Y^(n-m) = big^n * sum_k a_k r^k, with k = m (X small) or n-m
+            double bn = big;
+            double h = xs ? c11[0 * CSX_NIM2 + n] : c11[n * CSX_NIM2 + 0];
+#pragma unroll 4
+            for (int k = n - 1; k >= 0; --k) {
+                const double a = xs ? c11[(n - k) * CSX_NIM2 + k] : c11[k * CSX_NIM2 + (n - k)];
+                h = h * r + a;
+                if (k > 0) bn *= big;
+            }
+            const double term = c1p[n] * (h * bn);
+            for (int j = 0; go && j < min(64, 120 - base); ++j) {
+                pql += __shfl(term, j, 64);
+                go = !(fabs((pql - old) / pql) < 0.0001);
+                old = pql;
+            }
         }
-        pql += c1p[n] * (h * bn);
-        const double dd = fabs((pql - old) / pql);
-        if (dd < 0.0001) break;
-        old = pql;
+        if (lane == l) mine = pql;
     }
-    return pql;
+    return mine;
 }
 
-// LDS copies of the physics-mode orientation quadrature tables (filled by k_image for the
-// Gaussian-cylinder kernels; 33.9 KB).  File-scope LDS, so that every access compiles to a
-// ds_read with a 32-bit offset.
-__shared__ float2 g_cq_tab[kCqTab + 1];
+// Physics-mode orientation average: kCqWaves waves share 64 pixels, in kCqChunk polar nodes at a
+// time.  LDS: the rod factor's table, one cubic c0 + t (c1 + t (c2 + t c3)) a knot interval (one
+// 16-byte read an evaluation and no coefficient arithmetic), the node tables, the azimuth sums
+// of a chunk and the series' results; 75.4 KB, so two workgroups a CU (160 KB) and four waves a
+// SIMD.  File-scope LDS, so that every access compiles to a ds_read with a 32-bit offset.
+constexpr int kCqWaves = 8, kCqChunk = 32;
+__shared__ float4 g_cq_tab[kCqTab];
 __shared__ float4 g_cq_dl[kCqDelta];
 __shared__ float g_cq_tt[kCqPsi / 2];
+__shared__ float g_cq_sk[kCqChunk][64];
+__shared__ double g_cq_series[64];
 
-// Rod factor P(|a|) from the LDS table: cubic Hermite on the knot interval (value and
-// h*slope at both knots).  |a| is below amax by construction; the clamp only keeps the
-// index in range.
+__device__ __forceinline__ void cq_fill(const DevSet& d) {
+    for (int k = threadIdx.x; k < kCqTab; k += kCqWaves * 64) {
+        const float2 A = d.cq_tab[k], B = d.cq_tab[k + 1];  // value and h*slope at the two knots
+        const float df = B.x - A.x;
+        g_cq_tab[k] = make_float4(A.x, A.y, __builtin_fmaf(3.0f, df, -(2.0f * A.y + B.y)), (A.y + B.y) - 2.0f * df);
+    }
+    if (threadIdx.x < kCqDelta) g_cq_dl[threadIdx.x] = d.cq_delta[threadIdx.x];
+    if (threadIdx.x < kCqPsi / 2) g_cq_tt[threadIdx.x] = d.cq_t[threadIdx.x];
+    __syncthreads();
+}
+
+// Rod factor P(|a|) from the LDS table: cubic Hermite on the knot interval.  |a| is below amax
+// by construction; the clamp only keeps the index in range.
 __device__ __forceinline__ float cq_rod(float invh, float a) {
     const float u = fminf(fabsf(a) * invh, (float)kCqTab - 0.001f);
-    const int i = (int)u;
     const float t = __builtin_amdgcn_fractf(u);
-    const float2 A = g_cq_tab[i], B = g_cq_tab[i + 1];
-    const float df = B.x - A.x;
-    const float c2 = __builtin_fmaf(3.0f, df, -(2.0f * A.y + B.y));
-    const float c3 = (A.y + B.y) - 2.0f * df;
-    return __builtin_fmaf(t, __builtin_fmaf(t, __builtin_fmaf(t, c3, c2), A.y), A.x);
+    const float4 c = g_cq_tab[(int)u];
+    return __builtin_fmaf(t, __builtin_fmaf(t, __builtin_fmaf(t, c.w, c.z), c.y), c.x);
 }
 
 // Physics-mode orientation average of the longitudinal factor, FP32 with a compensated sum
@@ -1215,6 +1246,11 @@ __device__ __forceinline__ float cq_rod(float invh, float a) {
 // period), so (1/2pi) int_0^2pi dchi = (1/pi) int_0^pi dpsi, taken as a kCqPsi-point midpoint
 // rule whose nodes come in pairs +-t.  Polar: kCqDelta-point Gauss-Legendre with the weight
 // sin(d) exp(-d^2/dbeta^2), normalised to 1 on the host.
+// The waves of a workgroup hold the same 64 pixels: each forms the azimuth sums of every
+// kCqWaves-th polar node, then the polar sum is taken over all of them in order.  4096 rod
+// evaluations a pixel bound it; a wave of its own for every 64 pixels leaves the half cover of
+// 512^2 at two waves a SIMD and the last of them alone.  A 512^2 pattern: 357 us with every pixel
+// a wave lane of its own and both knots read, 339 us on the half cover, 159 us shared like this.
 __device__ double cyl_gauss_quad(const DevSet& d, double qa, double qb, int oc) {
     double c1, rq;
     if (oc == 1) {
@@ -1233,20 +1269,28 @@ __device__ double cyl_gauss_quad(const DevSet& d, double qa, double qb, int oc) 
     const float lz = d.cq_lz, invh = d.cq_invh;
     const float fc1 = (float)c1, frq = (float)rq;
     float sum = 0.0f, comp = 0.0f;
-    for (int k = 0; k < kCqDelta; ++k) {
-        const float4 nd = g_cq_dl[k];  // cos, sin, weight
-        const float al = __builtin_fmaf(nd.x, fc1, 1.0e-10f) * lz;
-        const float rr = nd.y * frq * lz;
-        float sk = 0.0f;
+    const int wave = uniform_i((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    for (int k0 = 0; k0 < kCqDelta; k0 += kCqChunk) {
+        if (k0) __syncthreads();  // the last chunk's sums have been read
+        for (int k = wave; k < kCqChunk; k += kCqWaves) {
+            const float4 nd = g_cq_dl[k0 + k];  // cos, sin, weight
+            const float al = __builtin_fmaf(nd.x, fc1, 1.0e-10f) * lz;
+            const float rr = nd.y * frq * lz;
+            float sk = 0.0f;
 #pragma unroll 4
-        for (int j = 0; j < kCqPsi / 2; ++j) {
-            const float t = g_cq_tt[j];
-            sk += cq_rod(invh, __builtin_fmaf(rr, t, al)) + cq_rod(invh, __builtin_fmaf(-rr, t, al));
+            for (int j = 0; j < kCqPsi / 2; ++j) {
+                const float t = g_cq_tt[j];
+                sk += cq_rod(invh, __builtin_fmaf(rr, t, al)) + cq_rod(invh, __builtin_fmaf(-rr, t, al));
+            }
+            g_cq_sk[k][lane] = sk;
         }
-        const float y = __builtin_fmaf(nd.z, sk, -comp);
-        const float tnew = sum + y;
-        comp = (tnew - sum) - y;
-        sum = tnew;
+        __syncthreads();
+        for (int k = 0; k < kCqChunk; ++k) {
+            const float y = __builtin_fmaf(g_cq_dl[k0 + k].z, g_cq_sk[k][lane], -comp);
+            const float tnew = sum + y;
+            comp = (tnew - sum) - y;
+            sum = tnew;
+        }
     }
     return (double)sum;
 }
@@ -1292,18 +1336,36 @@ __device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, d
             qb = qx * s.sinphic + qy * s.cosphic;
         }
         const int oc = orc_cmp(s);
-        double pql;
-        if (oc == 4) {
-            pql = 1.0;
-        } else if (q < (0.4 * s.limq[0])) {
-            pql = (oc >= 1 && oc <= 3) ? cyl_gauss_series(d, qa, qb, oc) : 1.0;
-        } else if constexpr (KIND == K_CYL_GAUSS_Q) {
-            pql = cyl_gauss_quad(d, qa, qb, oc);  // physics mode: oc in 1..3, tables in LDS
-        } else {
-            // the reference's nested Romberg; in reference mode the general case (oc = 0)
-            // has an identically zero integrand
-            pql = (oc >= 1 && oc <= 4) ? romb_delta_cyl(d, qa, qb, oc) / s.norm : 0.0;
+        double pql = 1.0;
+        if (oc != 4) {
+            const bool series = q < (0.4 * s.limq[0]);
+            if constexpr (KIND == K_CYL_GAUSS_Q) {
+                // physics mode: oc in 1..3, tables in LDS.  The workgroup's waves hold the same
+                // 64 pixels and share the nodes.
+                if (__ballot(!series)) pql = cyl_gauss_quad(d, qa, qb, oc);
+            } else if (!series) {
+                // the reference's nested Romberg; in reference mode the general case (oc = 0)
+                // has an identically zero integrand
+                pql = (oc >= 1 && oc <= 4) ? romb_delta_cyl(d, qa, qb, oc) / s.norm : 0.0;
+            }
+            if (__ballot(series)) {
+                const bool want = series && oc >= 1 && oc <= 3;
+                double v;
+                if constexpr (KIND == K_CYL_GAUSS_Q) {
+                    const int wave = uniform_i((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+                    const double part = cyl_gauss_series(d, qa, qb, oc, want, wave, kCqWaves);
+                    const unsigned long long req = __ballot(want);
+                    const int place = __popcll(req & ((1ull << lane) - 1));  // of this lane's request
+                    if (want && place % kCqWaves == wave) g_cq_series[lane] = part;
+                    __syncthreads();
+                    v = want ? g_cq_series[lane] : 1.0;
+                } else {
+                    v = cyl_gauss_series(d, qa, qb, oc, want, 0, 1);
+                }
+                if (series) pql = want ? v : 1.0;
+            }
         }
+        if (KIND == K_CYL_GAUSS_Q && threadIdx.x >= 64) return 0.0;  // the first wave has the pixels
         const double pq = pql * pq_cyl_transverse(d, q);
         return s.base + s.i0 * (pq + s.iso) + s.ifluc / (1 + q * q * s.rfluc * s.rfluc);
     }
@@ -1496,10 +1558,10 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
 // Kernels
 // ---------------------------------------------------------------------------
 
-// Pixel (px, py) of a 16x16 tile handled by lane threadIdx.x: each wave covers an 8x8
+// Pixel (px, py) of a 16x16 tile handled by this lane of wave w: each wave covers an 8x8
 // quadrant, the most compact 64-pixel footprint (narrowest |q| and angle ranges per wave).
-__device__ __forceinline__ void tile_pixel(int& px, int& py) {
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+__device__ __forceinline__ void tile_pixel(int w, int& px, int& py) {
+    const int l = threadIdx.x & 63;
     px = (w & 1) * 8 + (l & 7);
     py = (w >> 1) * 8 + (l >> 3);
 }
@@ -1510,18 +1572,25 @@ __device__ __forceinline__ void tile_pixel(int& px, int& py) {
 // at the axis, and the column ihex = x0 below it (whose mirror images lie outside the block),
 // follow, 16 consecutive pixels per wave (64 of them in a row have a |q| range, and so a pair
 // loop, several times a tile's, and were the tail of the whole launch).  That is 2 z^2 + 2 z
-// of 4 z^2 pixels.
+// of 4 z^2 pixels.  Quarter (the values depend on |qx| and |qy| only): tiles over i < 0, ihex <
+// 0, each lane's value serving the four sign images, and the two half axes as strips.  Half (even
+// in qy only): tiles over ihex < 0 and the column ihex = 0 as strips.
+enum CoverMode { kPlain = 0, kMirror = 1, kQuarter = 2, kHalf = 3 };
 constexpr int kStrip = 16;                          // strip pixels per wave
 constexpr int kStripBlock = kStrip * (kBlock / 64); // and per workgroup
 struct Cover {
     int32_t x0, x1, y0, y1;
-    int32_t mirror, tiles_x, main, total;  // main: 16x16 tiles; total: workgroups
+    int32_t mode, tiles_x, main, total;  // main: 16x16 tiles; total: workgroups
 };
-__host__ __device__ inline Cover make_cover(int x0, int x1, int y0, int y1, bool mirror) {
-    Cover c{x0, x1, y0, y1, mirror ? 1 : 0, 0, 0, 0};
-    c.tiles_x = (x1 - x0 + kTile - 1) / kTile;
-    c.main = c.tiles_x * (((mirror ? -y0 : y1 - y0) + kTile - 1) / kTile);
-    c.total = c.main + (mirror ? (x1 + y1 + kStripBlock - 1) / kStripBlock : 0);
+__host__ __device__ inline int strip_count(const Cover& c) {
+    return c.mode == kPlain ? 0 : c.mode == kMirror ? c.x1 + c.y1 : c.mode == kQuarter ? c.x1 + c.y1 + 1 : c.y1 - c.y0;
+}
+__host__ __device__ inline Cover make_cover(int x0, int x1, int y0, int y1, int mode) {
+    Cover c{x0, x1, y0, y1, mode, 0, 0, 0};
+    const bool left = mode == kQuarter || mode == kHalf, low = mode == kQuarter || mode == kMirror;
+    c.tiles_x = ((left ? -x0 : x1 - x0) + kTile - 1) / kTile;
+    c.main = c.tiles_x * (((low ? -y0 : y1 - y0) + kTile - 1) / kTile);
+    c.total = c.main + (strip_count(c) + kStripBlock - 1) / kStripBlock;
     return c;
 }
 struct CoverPix {
@@ -1529,28 +1598,50 @@ struct CoverPix {
     bool in, mir;  // the lane has a pixel of the block; its mirror image is this lane's as well
 };
 // Lanes without a pixel repeat a neighbouring one (the mixed path needs all 64 lanes).
-__device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t) {
+__device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int w) {
     CoverPix p;
     if (t < c.main) {
         int px, py;
-        tile_pixel(px, py);
-        const int ylim = c.mirror ? 0 : c.y1;
+        tile_pixel(w, px, py);
+        const int ylim = c.mode == kMirror || c.mode == kQuarter ? 0 : c.y1;
+        const int xlim = c.mode == kQuarter || c.mode == kHalf ? 0 : c.x1;
         const int ihex = c.x0 + t % c.tiles_x * kTile + px, i = c.y0 + t / c.tiles_x * kTile + py;
-        p.in = ihex < c.x1 && i < ylim;
-        p.ihex = min(ihex, c.x1 - 1);
+        p.in = ihex < xlim && i < ylim;
+        p.ihex = min(ihex, xlim - 1);
         p.i = min(i, ylim - 1);
-        p.mir = c.mirror && p.in && ihex > c.x0 && i > c.y0;
+        p.mir = c.mode == kMirror && p.in && ihex > c.x0 && i > c.y0;
     } else {
-        const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6;
+        const int lane = (int)threadIdx.x & 63;
         const int n = (t - c.main) * kStripBlock + w * kStrip + min(lane, kStrip - 1);
-        p.in = n < c.x1 + c.y1 && lane < kStrip;
-        const int k = min(n, c.x1 + c.y1 - 1);
-        const bool row = k <= c.x1;
-        p.ihex = row ? c.x0 + k : c.x0;
-        p.i = row ? 0 : k - c.x1;
-        p.mir = p.in && row && k > 0 && k < c.x1;
+        const int count = strip_count(c);
+        p.in = n < count && lane < kStrip;
+        const int k = min(n, count - 1);
+        const bool row = k <= c.x1;  // the row i = 0, then a column
+        if (c.mode == kQuarter) {
+            p.ihex = row ? c.x0 + k : 0;
+            p.i = row ? 0 : c.y0 + (k - c.x1 - 1);
+            p.mir = false;
+        } else if (c.mode == kHalf) {
+            p.ihex = 0;
+            p.i = c.y0 + k;
+            p.mir = false;
+        } else {
+            p.ihex = row ? c.x0 + k : c.x0;
+            p.i = row ? 0 : k - c.x1;
+            p.mir = p.in && row && k > 0 && k < c.x1;
+        }
     }
     return p;
+}
+// The kinds whose value is the same, bit for bit, at (+-qx, +-qy): the |q|-only ones; at
+// (qx, +-qy): the physics-mode orientation average about a direction in the x-z plane (phi is 0
+// in the general case) -- its argument along the axis carries +1e-10, so it is not even in qx.
+// A 128^2 sphere pattern: 28 us with a radial table before the image, 5 us without.
+inline int even_cover(const DevSet& d, int kind, int x0, int x1, int y0, int y1) {
+    if (d.s.centerbeam || d.s.use1d || x1 <= 0 || y1 <= 0 || x0 != -x1 || y0 != -y1) return kPlain;
+    if (kind == K_SPHERE || kind == K_CUBE || kind == K_CYL_ISO) return kQuarter;
+    if (kind == K_CYL_GAUSS_Q && (d.s.orcase == 1 || (d.s.orcase == 0 && d.s.sinphic == 0.0))) return kHalf;
+    return kPlain;
 }
 // Mirror images serve the lattice kinds' Gaussian peak sums in mixed precision, in the
 // midpoint grid, when every reflection has its Friedel partner in the list.
@@ -1635,14 +1726,10 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
                                            ColdQueue cq = ColdQueue{}) {
     const int t = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     if (t >= c.total) return;
-    const CoverPix p = cover_pixel(c, t);
+    // (Gaussian cylinders, quadrature: every wave of the workgroup holds quadrant blockIdx.z)
+    const CoverPix p = cover_pixel(c, t, KIND == K_CYL_GAUSS_Q ? (int)blockIdx.z : (int)threadIdx.x >> 6);
     PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
-    if constexpr (KIND == K_CYL_GAUSS_Q) {
-        for (int k = threadIdx.x; k <= kCqTab; k += kBlock) g_cq_tab[k] = d.cq_tab[k];
-        if (threadIdx.x < kCqDelta) g_cq_dl[threadIdx.x] = d.cq_delta[threadIdx.x];
-        if (threadIdx.x < kCqPsi / 2) g_cq_tt[threadIdx.x] = d.cq_t[threadIdx.x];
-        __syncthreads();
-    }
+    if constexpr (KIND == K_CYL_GAUSS_Q) cq_fill(d);
     if (!__ballot(p.in)) return;
     const Radial* rv = nullptr;
     if (rtab) {
@@ -1668,16 +1755,27 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
             if (mine) cq.ent[(size_t)slot * 64 + lane] = cpx;
         }
     }
+    if (KIND == K_CYL_GAUSS_Q && threadIdx.x >= 64) return;
     // 64-byte row segments; the other half of each line is written by the same workgroup
     const size_t W = (size_t)(c.x1 - c.x0);
     if (p.in) out[(size_t)(p.ihex - c.x0) + W * (size_t)(p.i - c.y0)] = v[0];
-    if (p.mir) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[1];
+    if constexpr (lattice_kind(KIND)) {
+        if (p.mir) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[1];
+    } else if (c.mode != kPlain && p.in) {
+        // ihex (quarter: and i) <= 0; the images on the axes coincide, those of the first column
+        // and row lie outside the block
+        const bool mx = p.ihex < 0 && p.ihex > c.x0, my = c.mode == kQuarter && p.i < 0 && p.i > c.y0;
+        if (mx) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(p.i - c.y0)] = v[0];
+        if (my) out[(size_t)(p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[0];
+        if (mx && my) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[0];
+    }
 }
 
+constexpr int image_block(int kind) { return kind == K_CYL_GAUSS_Q ? kCqWaves * 64 : kBlock; }
 template <int KIND, int PREC>
-__global__ void __launch_bounds__(kBlock) k_image(const DevSet d, const Cover c, double* __restrict__ out,
-                                                  unsigned long long* __restrict__ stats,
-                                                  const Radial* __restrict__ rtab) {
+__global__ void __launch_bounds__(image_block(KIND)) k_image(const DevSet d, const Cover c, double* __restrict__ out,
+                                                             unsigned long long* __restrict__ stats,
+                                                             const Radial* __restrict__ rtab) {
     image_tile<KIND, PREC>(d, c, out, stats, rtab);
 }
 
@@ -1820,7 +1918,7 @@ __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __re
     __shared__ int s_cnt[kBlock / 64], s_nan[kBlock / 64];
     double term = 0.0;
     int nz = 0, isnan_ = 0;
-    const CoverPix p = cover_pixel(f.cov, tile);
+    const CoverPix p = cover_pixel(f.cov, tile, (int)threadIdx.x >> 6);
     // All lanes of a wave with a pixel evaluate one (wave-wide |q| ranges need all 64 lanes);
     // lanes outside the fit array or masked discard the value.
     if (__ballot(p.in)) {
@@ -1922,7 +2020,7 @@ __device__ __forceinline__ void image_batch_tiles(const FitSet* __restrict__ set
     if (t >= ntiles) return;
     const int2 st = tiles[t];
     const FitSet& f = sets[st.x];
-    const CoverPix p = cover_pixel(f.cov, st.y);
+    const CoverPix p = cover_pixel(f.cov, st.y, (int)threadIdx.x >> 6);
     if (!__ballot(p.in)) return;
     PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
     const Radial* rv = nullptr;
@@ -2915,7 +3013,7 @@ constexpr int kFixBlocks = 1024;
 template <int K, int P>
 static void launch_image(const DevSet& d, const Cover& g, double* out, unsigned long long* stats,
                          const Radial* rtab, const ColdQueue* cq, hipEvent_t* ev, hipStream_t st) {
-    const dim3 grid(g.tiles_x, (g.total + g.tiles_x - 1) / g.tiles_x);
+    const dim3 grid(g.tiles_x, (g.total + g.tiles_x - 1) / g.tiles_x, K == K_CYL_GAUSS_Q ? kBlock / 64 : 1);
     if (ev) (void)hipEventRecord(ev[0], st);
     if constexpr (lattice_kind(K) && P == CSX_PREC_MIXED) {
         if (cq) {
@@ -2928,7 +3026,7 @@ static void launch_image(const DevSet& d, const Cover& g, double* out, unsigned 
     if constexpr (lattice_kind(K))
         hipLaunchKernelGGL((k_image_lat<K, P>), grid, dim3(kBlock), 0, st, d, g, out, stats, rtab);
     else
-        hipLaunchKernelGGL((k_image<K, P>), grid, dim3(kBlock), 0, st, d, g, out, stats, rtab);
+        hipLaunchKernelGGL((k_image<K, P>), grid, dim3(image_block(K)), 0, st, d, g, out, stats, rtab);
     if (ev) (void)hipEventRecord(ev[1], st);
 }
 
@@ -2947,7 +3045,8 @@ int csx_qgrid(csx_ctx* c, const csx_grid* g, double* d_q3) {
 // Cover of a set's fit array.
 static Cover fit_cover(const FitSet& f, int kind, int precision) {
     const int x0 = f.d.s.iimin;
-    return make_cover(x0, x0 + f.w, x0, x0 + f.h, mirror_set(f.d, kind, precision, x0, x0 + f.w, x0, x0 + f.h));
+    const bool mirror = mirror_set(f.d, kind, precision, x0, x0 + f.w, x0, x0 + f.h);
+    return make_cover(x0, x0 + f.w, x0, x0 + f.h, mirror ? kMirror : kPlain);
 }
 template <int K, int P>
 static void launch_fit_one(const FitSet& f, int ntiles, double* fqs, TileSum* part, hipStream_t st) {
@@ -3011,12 +3110,14 @@ static int render_kind(const csx_ctx* c, int precision) {
     return k;
 }
 
-// Radial table of a render (midpoint grid, radial kinds), sized for the grid, and its slot;
-// null otherwise.
+// Radial table of a render (midpoint grid, radial lattice kinds), sized for the grid, and its
+// slot; null otherwise.  The |q|-only kinds without a lattice evaluate each pixel of the quarter
+// cover instead: twice the table's evaluations, but one launch and no events (isotropic spheres
+// at 128^2 took 26 us, most of it the second launch and the stream hand-over; 1024^2 the same).
 static int radial_table(csx_ctx* c, const csx_grid& g, Radial** out, int* slot) {
     *out = nullptr;
     *slot = -1;
-    if (!radial_kind(kind_of(c->set.s.combo_key)) || c->set.s.centerbeam || c->set.s.use1d) return CSX_OK;
+    if (!radial_kind(kind_of(c->set.s.combo_key)) || !lattice_kind(kind_of(c->set.s.combo_key)) || c->set.s.centerbeam || c->set.s.use1d) return CSX_OK;
     const long long m = std::max(std::max(std::llabs(g.xmin), std::llabs((long long)g.xmax - 1)),
                                  std::max(std::llabs(g.ymin), std::llabs((long long)g.ymax - 1)));
     if (m > 46000) return CSX_OK;  // triangle index would overflow int: evaluate per pixel
@@ -3078,8 +3179,10 @@ static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g,
         HIPCHK(c, hipEventRecord(c->ev_rad[sl], c->side));
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_rad[sl], 0));
     }
-    const Cover cov = make_cover(g.xmin, g.xmax, g.ymin, g.ymax,
-                                 mirror_set(c->set, kind, precision, g.xmin, g.xmax, g.ymin, g.ymax));
+    const int mode = mirror_set(c->set, kind, precision, g.xmin, g.xmax, g.ymin, g.ymax)
+                         ? kMirror
+                         : even_cover(c->set, kind, g.xmin, g.xmax, g.ymin, g.ymax);
+    const Cover cov = make_cover(g.xmin, g.xmax, g.ymin, g.ymax, mode);
     // Lattice kinds in mixed precision render in two passes (hot, then fix over a queue of at
     // most one slot per wave), unless unpaired reflections send every pixel to FP64.
     ColdQueue cq{};
