@@ -209,29 +209,23 @@ __global__ void k_rphi(const double* __restrict__ imgs, RphiArgs a, const RphiIm
 }
 
 // ---- FFT image (calculateIFFT without FFTW, Source/sc_postproc.cpp:364-560, 833-1000) ----
-// One workgroup per line of the 2D transform (rows of one pass, columns of the other), the
-// line in LDS: bit-reversal permutation on load, then the butterfly levels.  The twiddles are
-// the reference's recurrence, evaluated on the host in the same order and passed in a table
-// (level l, l1 = 2^l entries from index l1 - 1), so every butterfly rounds as there.
-__global__ void k_fft_lines(double2* __restrict__ buf, int64_t img_stride, int64_t line_stride, int64_t elem_stride,
-                            int m, const double2* __restrict__ tw, int forward) {
-    extern __shared__ double lds[];
+// Both passes: a workgroup transforms G neighbouring lines in LDS, bit-reversal permutation on
+// load, then the butterfly levels.  The twiddles are the reference's recurrence, evaluated on the
+// host in the same order and passed in a table (level l, l1 = 2^l entries from index l1 - 1), so
+// every butterfly rounds as there.  Memory bounds it: line g of a workgroup starts g places
+// into its LDS row and wraps, so that reads along the lines and across them both spread over the banks,
+// and both passes read and write G neighbouring elements at a time.
+__device__ __forceinline__ int fft_slot(int nn, int g, int i) { return g * nn + ((i + g) & (nn - 1)); }
+
+__device__ __forceinline__ void fft_levels(double* xr, double* xi, int m, int lines, const double2* __restrict__ tw) {
     const int nn = 1 << m;
-    double* xr = lds;
-    double* xi = lds + nn;
-    double2* line = buf + (int64_t)blockIdx.y * img_stride + (int64_t)blockIdx.x * line_stride;
-    for (int i = threadIdx.x; i < nn; i += blockDim.x) {
-        const int r = (int)(__brev((unsigned)i) >> (32 - m));
-        const double2 v = line[(int64_t)r * elem_stride];
-        xr[i] = v.x;
-        xi[i] = v.y;
-    }
     __syncthreads();
     for (int l = 0; l < m; ++l) {
         const int l1 = 1 << l, l2 = l1 << 1;
-        for (int b = threadIdx.x; b < nn / 2; b += blockDim.x) {
+        for (int e = threadIdx.x; e < lines * (nn / 2); e += blockDim.x) {
+            const int g = e >> (m - 1), b = e & (nn / 2 - 1);
             const int jj = b & (l1 - 1);
-            const int i = (b >> l) * l2 + jj, i1 = i + l1;
+            const int k = (b >> l) * l2 + jj, i = fft_slot(nn, g, k), i1 = fft_slot(nn, g, k + l1);
             const double2 u = tw[l1 - 1 + jj];
             const double t1 = u.x * xr[i1] - u.y * xi[i1];
             const double t2 = u.x * xi[i1] + u.y * xr[i1];
@@ -242,24 +236,39 @@ __global__ void k_fft_lines(double2* __restrict__ buf, int64_t img_stride, int64
         }
         __syncthreads();
     }
-    for (int i = threadIdx.x; i < nn; i += blockDim.x) {
-        double a = xr[i], b = xi[i];
+}
+
+// Lines of one workgroup at size s: 256 bytes of neighbouring complex elements, in at most 64 KB
+// of LDS.  One column a workgroup (16 bytes of each line of memory) took 131 us for 256 images of
+// 128^2, where the contiguous pass took 31; load, both passes and output together 225 -> 71 us.
+inline int fft_lines(int s) { return std::min(std::min(s, 16), 4096 / s); }
+
+// First pass, along the first index (stride s): c[y][x] = d[x + s y] / max, imaginary part 0,
+// transformed, to buf.
+__global__ void __launch_bounds__(512) k_fft_first(const double* __restrict__ d, const double* __restrict__ mx,
+                                                   double2* __restrict__ buf, int m, int lines,
+                                                   const double2* __restrict__ tw, int forward) {
+    extern __shared__ double lds[];
+    const int nn = 1 << m, x0 = blockIdx.x * lines, lg = __builtin_ctz(lines);
+    double *xr = lds, *xi = lds + lines * nn;
+    const int64_t base = (int64_t)blockIdx.y * nn * nn + x0;
+    const double mv = mx[blockIdx.y];
+    for (int e = threadIdx.x; e < lines * nn; e += blockDim.x) {
+        const int g = e & (lines - 1), r = e >> lg;
+        const int at = fft_slot(nn, g, (int)(__brev((unsigned)r) >> (32 - m)));
+        xr[at] = d[base + (int64_t)r * nn + g] / mv;
+        xi[at] = 0.0;
+    }
+    fft_levels(xr, xi, m, lines, tw);
+    for (int e = threadIdx.x; e < lines * nn; e += blockDim.x) {
+        const int g = e & (lines - 1), r = e >> lg, at = fft_slot(nn, g, r);
+        double a = xr[at], b = xi[at];
         if (forward) {
             a /= (double)nn;
             b /= (double)nn;
         }
-        line[(int64_t)i * elem_stride] = make_double2(a, b);
+        buf[base + (int64_t)r * nn + g] = make_double2(a, b);
     }
-}
-
-// Input of the transform: c[y][x] = d[x + s y] / max, imaginary part 0.
-__global__ void k_fft_load(const double* __restrict__ d, int64_t len, const double* __restrict__ mx,
-                           double2* __restrict__ buf) {
-    const double* src = d + (int64_t)blockIdx.y * len;
-    double2* dst = buf + (int64_t)blockIdx.y * len;
-    const double m = mx[blockIdx.y];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = make_double2(src[i] / m, 0.0);
 }
 
 // Output cell (x, y) takes c[x][y] (the reference reads the array transposed) at
@@ -275,25 +284,44 @@ __device__ __forceinline__ int64_t fft_index(int swap, int x, int y, int dim) {
     return x + (int64_t)dim * y;
 }
 
-__global__ void k_fft_out(const double2* __restrict__ buf, int s, int out_type, int swap, double* __restrict__ out) {
-    const int64_t len = (int64_t)s * s;
-    const double2* c = buf + (int64_t)blockIdx.y * len;
+// Second pass, along the second index, and the output image from its lines: the transposed read
+// of the output would be strided again (48 us as a pass of its own, and the complex image written
+// and read once more).
+__global__ void __launch_bounds__(512) k_fft_second(const double2* __restrict__ buf, int m, int lines,
+                                                    const double2* __restrict__ tw, int forward, int out_type,
+                                                    int swap, double* __restrict__ out) {
+    extern __shared__ double lds[];
+    const int nn = 1 << m, x0 = blockIdx.x * lines, lg = __builtin_ctz(lines);
+    double *xr = lds, *xi = lds + lines * nn;
+    const int64_t len = (int64_t)nn * nn;
+    const double2* c = buf + (int64_t)blockIdx.y * len + (int64_t)x0 * nn;
     double* o = out + (int64_t)blockIdx.y * len;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < len; k += (int64_t)gridDim.x * blockDim.x) {
-        const int y = (int)(k / s), x = (int)(k % s);
+    for (int e = threadIdx.x; e < lines * nn; e += blockDim.x) {
+        const int at = fft_slot(nn, e >> m, (int)(__brev((unsigned)(e & (nn - 1))) >> (32 - m)));
+        const double2 v = c[e];
+        xr[at] = v.x;
+        xi[at] = v.y;
+    }
+    fft_levels(xr, xi, m, lines, tw);
+    for (int e = threadIdx.x; e < lines * nn; e += blockDim.x) {
+        const int g = e & (lines - 1), y = e >> lg, x = x0 + g, at = fft_slot(nn, g, y);
         if (swap && (x == 0 || y == 0)) {
-            o[k] = 0.0;  // cell (0, k) or (k, 0) of the output: never written
+            o[x + (int64_t)nn * y] = 0.0;  // cell (0, k) or (k, 0) of the output: never written
             continue;
         }
-        const double2 v = c[(int64_t)x * s + y];
+        double a = xr[at], b = xi[at];
+        if (forward) {
+            a /= (double)nn;
+            b /= (double)nn;
+        }
         double r;
         switch (out_type) {
-        case 0: r = v.x; break;
-        case 1: r = v.y; break;
-        case 2: r = sqrt(v.x * v.x + v.y * v.y); break;
-        default: r = (v.x + v.y) * (v.x - v.y); break;
+        case 0: r = a; break;
+        case 1: r = b; break;
+        case 2: r = sqrt(a * a + b * b); break;
+        default: r = (a + b) * (a - b); break;
         }
-        o[fft_index(swap, x, y, s)] = r;
+        o[fft_index(swap, x, y, nn)] = r;
     }
 }
 
@@ -674,15 +702,12 @@ int csx_post_ifft(csx_ctx* c, const double* d_in, int s, int nimg, int forward, 
     hipStream_t st = (hipStream_t)csx_ctx_stream(c);
     PCHK(c, hipMemcpyAsync(d_tw, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_max0, dim3(nimg), dim3(kStat), 0, st, d_in, len, mx);
-    hipLaunchKernelGGL(k_fft_load, dim3(blocks_for(len), nimg), dim3(256), 0, st, d_in, len, mx, buf);
-    const int threads = std::min(1024, std::max(64, s / 2));
-    const size_t shm = 2 * (size_t)s * sizeof(double);
-    // along the first index (stride s) for every second index, then along the second
-    hipLaunchKernelGGL(k_fft_lines, dim3(s, nimg), dim3(threads), shm, st, buf, len, (int64_t)1, (int64_t)s, m, d_tw,
+    const int lines = fft_lines(s), threads = std::min(512, std::max(64, lines * s / 2));
+    const size_t shm = 2 * (size_t)lines * s * sizeof(double);
+    hipLaunchKernelGGL(k_fft_first, dim3(s / lines, nimg), dim3(threads), shm, st, d_in, mx, buf, m, lines, d_tw,
                        forward);
-    hipLaunchKernelGGL(k_fft_lines, dim3(s, nimg), dim3(threads), shm, st, buf, len, (int64_t)s, (int64_t)1, m, d_tw,
-                       forward);
-    hipLaunchKernelGGL(k_fft_out, dim3(blocks_for(len), nimg), dim3(256), 0, st, buf, s, out_type, swap, full);
+    hipLaunchKernelGGL(k_fft_second, dim3(s / lines, nimg), dim3(threads), shm, st, buf, m, lines, d_tw, forward,
+                       out_type, swap, full);
     PCHK(c, hipGetLastError());
     // (its maxima go to the start of scratch 1, which mx no longer needs; the twiddles and
     // the full image lie past them)

@@ -178,6 +178,23 @@ def test_fft_matches_the_reference(name):
         assert err < 1e-13
 
 
+@pytest.mark.parametrize("s", [4, 8, 16, 32, 128, 256, 512, 1024, 2048])
+@pytest.mark.parametrize("forward,out_type,swap", [(0, 2, True), (1, 0, False)])
+def test_fft_sizes(oracle_lib, s, forward, out_type, swap):
+    """Sizes from one workgroup an image (4) to two lines a workgroup (2048), against the oracle.
+    The levels round as there; a transform sums s^2 values of about 1, so an output differs by at
+    most some ulps of that sum's terms: 1e-13 of the largest."""
+    import torch
+    from crystalscatter_amd import aidata
+    n = 2
+    d = np.random.default_rng(s).random((n, s * s)) + 0.1
+    x = torch.from_numpy(d).cuda()
+    got = aidata.post_ifft(Context(0), x, s, forward, out_type, scale=False, swap=swap).cpu().numpy().reshape(n, -1)
+    for k in range(n):
+        want = oracle_lib.ifft(d[k], s, forward, out_type, swap=swap).ravel()
+        assert np.abs(got[k] - want).max() <= 1e-13 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("name,lin", [("fcc_rphi", 0), ("sphere_lin", 1)])
 def test_scale_intensity_matches_the_reference(name, lin):
     import torch
