@@ -1,8 +1,8 @@
 // csx_device.hip -- HIP kernels (gfx950) and the device half of the C ABI.
 //
-// One thread per detector pixel, 16x16-pixel tiles per 256-thread block
-// (4 wave64s, each a 16x4 strip), coalesced FP64 stores in the reference's IDX
-// order.  Per-pixel form factors run in FP64 with the reference formulas; the
+// One lane per detector pixel, or per pixel and its symmetric images (Cover),
+// 16x16-pixel tiles per 256-thread block (4 wave64s, each an 8x8 quadrant),
+// FP64 stores in the reference's IDX order.  Per-pixel form factors run in FP64 with the reference formulas; the
 // Gaussian peak sums run either in FP64 exactly as the reference writes them
 // (CSX_PREC_REF64) or in FP32 over Friedel pairs (CSX_PREC_MIXED): +hkl and
 // -hkl share |q^.u| and |q_hkl|, so one acos/sqrt serves both, their angular
