@@ -55,14 +55,17 @@ constexpr int64_t kOutW = w_off(kL);
 constexpr int64_t kOutB = kOutW + kH;
 constexpr int64_t kNParams = kOutB + 1;
 
-// Sigmoid from the hardware exp2 and reciprocal (1 ulp each): the activations are stored in
-// bf16, and an IEEE division here was a third of the inference's instructions.
+// Sigmoid 1 / (1 + e^-z): the reciprocal of the hardware, 1 ulp, with one Newton step, which
+// rounds it correctly; an IEEE division here was a third of the inference's instructions.  The
+// denominator is kept finite, so that the step of an infinite one gives 0 like the division.
 __device__ __forceinline__ float sigm(float z) {
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950409f * z));
+    const float x = fminf(1.0f + __expf(-z), 3.402823466e38f);
+    const float r = __builtin_amdgcn_rcpf(x);
+    return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
 __device__ __forceinline__ float silu_grad(float z) {
     const float s = sigm(z);
-    return s * __builtin_fmaf(z, 1.0f - s, 1.0f);
+    return s * (1.0f + z * (1.0f - s));
 }
 
 // Position of weight (row, k) of a [rows][K] matrix in its bf16 copy: MFMA A fragments of 16 rows
@@ -87,10 +90,12 @@ struct Features {
 // W . H^T (D[feature][row]): the weights are the A operand, read straight from the bf16
 // [out][in] copies (L2-resident), the rows' activations the B operand, from LDS.  A lane then
 // holds four consecutive features of one row, so the epilogue writes 8 bytes where the other
-// orientation writes four 2-byte values.  The bias is the accumulators' initial value.
-// Bound: the vector unit -- per row 1024 SiLU values at about 46 cycles each per wave of 64
-// (exp2 and reciprocal at quarter rate) against 422 matrix cycles.  2.1 M rows of inference:
-// 1.22 ms (2.72 ms with H . W^T, IEEE divisions and row-major weights); with 8 waves 1.32 ms.
+// orientation writes four 2-byte values.  The bias is added to the finished products.
+// Bound: the vector unit -- per row 1024 SiLU values at about 60 cycles each per wave of 64
+// (exp2 and reciprocal at quarter rate) and 32 sincosf, against 422 matrix cycles.  2.1 M rows of
+// inference: 1.26 ms (2.75 ms with H . W^T, IEEE divisions and row-major weights).  1.10 ms with
+// the bare reciprocal, hardware sines of the phase in turns and the bias as the accumulators'
+// initial value, but then activations flip bf16 roundings and y moves by 8e-4 in norm.
 // Training, 65,536 rows: 0.16 ms, its phases between barriers (4 waves at 2 per SIMD: 0.22 ms),
 // for the 11 launches and 0.38 ms of the layer-by-layer passes.
 constexpr int kPM = 64;        // rows per block
@@ -100,7 +105,7 @@ static_assert(kPM == 64 && kH == 256, "one lane per row");
 
 // Parameters of set[i] (already normalised by the caller; an index outside [0, nsets) is
 // clamped, the host checks them), then sin and cos of the kNF phases, then zeros; rows >= n are
-// zero.  Lane = row; each wave takes kNF / NW phases.  The phase is formed in turns.
+// zero.  Lane = row; each wave takes kNF / NW phases.
 template <int NW>
 __device__ __forceinline__ void embed_rows(int r0, int n, int nsets, const float* __restrict__ par,
                                            const int32_t* __restrict__ set, const float* __restrict__ q,
@@ -129,25 +134,23 @@ __device__ __forceinline__ void embed_rows(int r0, int n, int nsets, const float
     if (wave == 0)
 #pragma unroll
         for (int k = 0; k < kNP; k += 2) row[k / 2] = pack(v[k], v[k + 1]);
-    const float qa = sqrtf(qx * qx + qy * qy) * 0.15915494309f;  // turns
+    const float qa = sqrtf(qx * qx + qy * qy);
     constexpr int NF = kNF / NW;
-    float sn[NF], cs[NF];
-#pragma unroll
-    for (int f0 = 0; f0 < NF; ++f0) {
-        const int f = wave * NF + f0;
-        const int j = ft.pidx[f];
-        float pv = 1.0f;
-#pragma unroll
-        for (int k = 0; k < kNP; ++k) pv = (k == j) ? ft.off[k] + ft.sc[k] * v[k] : pv;
-        const float turn =
-            __builtin_amdgcn_fractf((ft.f[f][0] * qx + ft.f[f][1] * qy) + ft.f[f][2] * qa * pv);
-        sn[f0] = live ? __builtin_amdgcn_sinf(turn) : 0.0f;
-        cs[f0] = live ? __builtin_amdgcn_cosf(turn) : 0.0f;
-    }
-#pragma unroll
+#pragma unroll 1
     for (int f0 = 0; f0 < NF; f0 += 2) {
-        row[(kNP + NF * wave + f0) / 2] = pack(sn[f0], sn[f0 + 1]);
-        row[(kNP + kNF + NF * wave + f0) / 2] = pack(cs[f0], cs[f0 + 1]);
+        float sn[2], cs[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int f = wave * NF + f0 + e;
+            const int j = ft.pidx[f];
+            float pv = 1.0f;
+#pragma unroll
+            for (int k = 0; k < kNP; ++k) pv = (k == j) ? ft.off[k] + ft.sc[k] * v[k] : pv;
+            sincosf(6.283185307f * (ft.f[f][0] * qx + ft.f[f][1] * qy) + ft.f[f][2] * qa * pv, &sn[e], &cs[e]);
+            if (!live) sn[e] = cs[e] = 0.0f;
+        }
+        row[(kNP + NF * wave + f0) / 2] = pack(sn[0], sn[1]);
+        row[(kNP + kNF + NF * wave + f0) / 2] = pack(cs[0], cs[1]);
     }
     for (int k = kUsed / 2 + wave; k < kIn / 2; k += NW) row[k] = 0u;
 }
@@ -274,28 +277,29 @@ __global__ void __launch_bounds__(64 * NW, 4) k_mlp(int n, int nsets, const floa
         f32x4 acc[NI][4];
         const float* b = p + b_off(l);
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const f32x4 bi = {b[acc_feature(wn, i)], b[acc_feature(wn, i) + 1], b[acc_feature(wn, i) + 2],
-                              b[acc_feature(wn, i) + 3]};
+        for (int i = 0; i < NI; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = bi;
-        }
+            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         if (l == 0) layer_product<kIn, NI, !TRAIN>(wb, act, wn, acc);
         else layer_product<kH, NI, !TRAIN>(wb + kW1 + (l - 1) * kWl, act, wn, acc);
         __syncthreads();  // every wave has read the layer's input
+        __builtin_amdgcn_sched_barrier(0);  // the bias loads would be moved up here and spill
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int i = 0; i < NI; ++i) {
+            const float* bi = b + acc_feature(wn, i);
+            const float bias[4] = {bi[0], bi[1], bi[2], bi[3]};
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
+            for (int j = 0; j < 4; ++j) {
                 bf16x4 h;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float zz = acc[i][j][r];
+                    const float zz = acc[i][j][r] + bias[r];
                     h[r] = (bf16)(zz * sigm(zz));
                     if constexpr (TRAIN) z[l][i][j][r] = (bf16)zz;
                 }
                 *(bf16x4*)&act[acc_row(j) * kPLd + acc_feature(wn, i)] = h;
             }
+        }
         __syncthreads();
         if constexpr (TRAIN)
             if (l < kL - 1) store_columns<NW, false>(act, tr.ht[l] + (size_t)r0 * kH, kH, nullptr);
@@ -627,8 +631,8 @@ int check_rows(csx_mlp* m, int n, int nsets) {
 }
 
 int infer(csx_mlp* m, int n, int nsets, const float* d_par, const int32_t* d_set, const float* d_q, float* d_y) {
-    hipLaunchKernelGGL((k_mlp<false, kInferWaves>), dim3((unsigned)((n + kPM - 1) / kPM)), dim3(64 * kInferWaves), 0, m->stream, n, nsets, d_par,
-                       d_set, d_q, m->feat, m->wb, m->p, d_y, TrainArgs{});
+    hipLaunchKernelGGL((k_mlp<false, kInferWaves>), dim3((unsigned)((n + kPM - 1) / kPM)), dim3(64 * kInferWaves), 0,
+                       m->stream, n, nsets, d_par, d_set, d_q, m->feat, m->wb, m->p, d_y, TrainArgs{});
     MCHK(m, hipGetLastError());
     return CSX_OK;
 }
@@ -828,8 +832,8 @@ int csx_mlp_gradient(csx_mlp* m, int n, int nsets, const float* d_par, const int
         wg.part[l] = m->part + (l == 0 ? 0 : m->splits * (w1 + (l - 1) * wl));
         fa.part[l] = wg.part[l];
     }
-    hipLaunchKernelGGL((k_mlp<true, kTrainWaves>), dim3(nb), dim3(64 * kTrainWaves), 0, m->stream, n, nsets, d_par, d_set, d_q, m->feat, m->wb, m->p,
-                       (float*)nullptr, tr);
+    hipLaunchKernelGGL((k_mlp<true, kTrainWaves>), dim3(nb), dim3(64 * kTrainWaves), 0, m->stream, n, nsets, d_par,
+                       d_set, d_q, m->feat, m->wb, m->p, (float*)nullptr, tr);
     MCHK(m, hipGetLastError());
     wg.kchunk = (nb + m->splits - 1) / m->splits;
     const int ns = (nb + wg.kchunk - 1) / wg.kchunk;

@@ -162,3 +162,17 @@ def test_gradient_rows(n):
     lb, gb = mo.loss_and_grad(net.get_params().astype(np.float64), X, t, bf16=True)
     assert abs(loss - lb) <= 2e-2 * lb                           # bf16 activations: 8-bit mantissas
     assert np.linalg.norm(g - gb) <= 2e-2 * np.linalg.norm(gb)   # as for the whole batch
+
+
+@pytest.mark.parametrize("physics", [False, True])
+def test_forward_equals_recorded(physics):
+    """y of 1000 rows as the first kernels of this network computed it, one product per layer with
+    sincosf, an IEEE division in the sigmoid and the bias added to the sums.  The order of the
+    sums is the same, so only the last bits of y may differ: one bf16 activation off by a rounding
+    moves y by about 1e-4 of its scale."""
+    from helpers import fixture
+    net = _net(max_batch=1024, physics=physics)
+    (_, _, _, _), (dpar, dsets, dq, _) = _inputs(1000, seed=7)
+    y = net.forward(dpar, dsets, dq).cpu().numpy()
+    ref = fixture("mlp_forward.npz")["physics" if physics else "random"]
+    assert np.abs(y - ref).max() <= 1e-6 * np.abs(ref).max()
