@@ -382,30 +382,12 @@ __device__ inline double fq_cyl_zdir(const DevSet& d, double limql, double qxs, 
     return fq_cyl_long(d, limql, qxs, qys) * fq_cyl_radial(d, q);
 }
 
-// rod_p from the set's constants, for the mixed path, at the projection p + 1e-9 and, with two,
-// at its mirror image -p + 1e-9: the power by exp and log, one division.  On the line p = 0 the
-// power is exactly 1, as rod_p's.  The rod factor f is even, so f(-p + e) = f(p - e) =
-// f(p + e) - 2 e f'(p) + O(e^3), and with e = 1e-9 an FP32 slope leaves about 1e-13 of f: a
-// second evaluation, in a loop or inlined, took 70 registers or its own 250 operations.
-template <int NV>
-__device__ __forceinline__ void rod_p_fast(const DevSet& d, double p, double* out) {
+// rod_p from the set's constants, for the mixed path, at the projection p + 1e-9: the power by
+// exp and log, one division.  On the line p = 0 the power is exactly 1, as rod_p's.
+__device__ __forceinline__ double rod_p_fast(const DevSet& d, double p) {
     const double arg = (p + 0.000000001) * d.cyl_ll, a2 = arg * arg;
-    const double lb = log(1.0 + 4 * a2);
-    const double ph = d.cyl_zl1 * atan(2.0 * arg);
-    const double c = cos(ph), E = exp(-0.5 * d.cyl_zl1 * lb);
-    const double g = 1 - c * E;
-    const double ia2 = 1 / a2;
-    out[0] = d.cyl_rc * g * ia2;
-    if constexpr (NV > 1) {
-        // f = rc g / a^2, g = 1 - cos(ph) E: g' = E ph' (sin(ph) + 2 a cos(ph)), ph' = 2 n / (1 + 4 a^2)
-        const float a = (float)arg;
-        const float dph = (float)(2.0 * d.cyl_zl1) * __builtin_amdgcn_rcpf(__builtin_fmaf(4.0f * a, a, 1.0f));
-        const float sn = __builtin_amdgcn_sinf(__builtin_amdgcn_fractf((float)(ph * 0.15915494309189535)));
-        const float gp = (float)E * dph * __builtin_fmaf(2.0f * a, (float)c, sn);
-        const float slope = gp - 2.0f * (float)g * __builtin_amdgcn_rcpf(a);
-        out[1] = out[0] - 2.0e-9 * d.cyl_ll * d.cyl_rc * ia2 * (double)slope;
-        if (p == 0.0) out[1] = out[0];
-    }
+    const double E = exp(-0.5 * d.cyl_zl1 * log(1.0 + 4 * a2));
+    return d.cyl_rc * (1 - cos(d.cyl_zl1 * atan(2.0 * arg)) * E) * (1 / a2);
 }
 
 // pq_cyl_long_zdir and fq_cyl_long at one pixel: the same values (FAST: to rounding), with the
@@ -431,8 +413,19 @@ __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, do
     double rod[NV];
     for (int k = 0; k < NV; ++k) rod[k] = 0.0;
     if (!fser || (!pser && same)) {
-        if constexpr (FAST) rod_p_fast<NV>(d, p, rod);
-        else rod[0] = rod_p(zlf, (p + 0.000000001) * s.length / (zlf + 1));
+        if constexpr (FAST) {
+            // The factor is even but its argument carries +1e-9, so the mirror image's is another
+            // value unless p is 0 (all of a pattern of cylinders along the beam).  It is evaluated
+            // on its own: where p is not far above 1e-9 (the line across the rods, where p is a
+            // rounding error unless an axis lies on it) a step from p's value loses every digit.
+            rod[0] = rod_p_fast(d, p);
+            if constexpr (NV > 1) {
+                rod[1] = rod[0];
+                if (p != 0.0) rod[1] = rod_p_fast(d, -p);
+            }
+        } else {
+            rod[0] = rod_p(zlf, (p + 0.000000001) * s.length / (zlf + 1));
+        }
     }
     for (int k = 0; k < NV; ++k) {
         pl[k] = pser ? ps : rod[k];

@@ -42,6 +42,25 @@ def test_image_against_fp64(kind, z):
         assert rel_err(m[ok], r[ok]).max() <= 1e-4   # the mixed mode's bar for every pixel
 
 
+@pytest.mark.parametrize("theta,phi", [(30, 45), (60, 90), (30, 135), (90, 45), (60, -45), (45, 90), (180, 0), (37, 20)])
+@pytest.mark.parametrize("length,sigmal", [(3, 0.06), (10, 0.06), (30, 0.06), (40, 0.3)])
+def test_cylinders_off_the_axes(theta, phi, length, sigmal):
+    """Cylinders whose projection vanishes on a line of pixels only up to rounding (the cosine and
+    sine of 45 degrees differ by one ulp, the cosine of 90 is 6e-17; at theta = 180 on every
+    pixel): both images of each pixel against the FP64 mode."""
+    print(theta, phi, length, sigmal, flush=True)
+    p = dict(BCT, theta=theta, phi=phi, Length=length, SigmaL=sigmal)
+    e = _engine(p, 64)
+    r = e.doCalculation("ref64")
+    ok = np.isfinite(r) & (r != 0)
+    batch = render_batch(Context(0), [_engine(p, 64, -1)], "mixed")[0].cpu().numpy()
+    for m in (e.doCalculation("mixed"), batch):
+        assert np.array_equal(np.isfinite(m), np.isfinite(r))
+        err = rel_err(m[ok], r[ok])
+        at = np.flatnonzero(ok)[err.argmax()]
+        assert err.max() <= 1e-4, (err.max(), at % 128 - 64, at // 128 - 64, m[at], r[at])
+
+
 @pytest.mark.parametrize("kind", ["fcc", "bct_cylinder"])
 @pytest.mark.parametrize("z", [1, 8, 17, 33])
 def test_objective_terms(kind, z):
