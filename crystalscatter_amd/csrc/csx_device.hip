@@ -759,9 +759,10 @@ __device__ __forceinline__ void near_one_add(const DevSet& d, const Window& W, c
 // called by all 64 lanes of a wave: the wave's union of per-lane windows selects the pairs.
 // Pairs outside the window, and second Friedel terms where they cannot reach 2^cut, are
 // dropped: every dropped term is below 2^cut * A.  need_exact: unpaired reflections exist.
+// npx: the pixels that the lane's value serves (for the counts).
 template <bool PLANAR, bool PRECISE, int MODE = kFull>
 __device__ __forceinline__ double lattice_mixed(const DevSet& d, PixQ& P3, double q, double width, bool& need_exact,
-                                double& dropped, Window& W, unsigned long long* stats) {
+                                double& dropped, Window& W, int npx, unsigned long long* stats) {
     const csx_scalars& s = d.s;
     PixelConsts L;
     pixel_dirs(s, P3, q, L);
@@ -899,7 +900,7 @@ __device__ __forceinline__ double lattice_mixed(const DevSet& d, PixQ& P3, doubl
         atomicAdd(&stats[0], (unsigned long long)(64 * evals));
         atomicAdd(&stats[3], (unsigned long long)(any_two ? 1 : 0));
     }
-    if (MODE != kFix && stats && flag) atomicAdd(&stats[2], 1ull);
+    if (MODE != kFix && stats && flag) atomicAdd(&stats[2], (unsigned long long)npx);
     need_exact = d.nsingle > 0;
     return inten;
 }
@@ -1372,17 +1373,18 @@ __device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, d
 }
 
 // Value v[0] of the pixel P3 (its exact q vector is computed here unless the caller has it) and,
-// with `mir`, v[1] of its mirror image (-ihex, -i); rv: its radial-table entry (midpoint grid,
-// radial kinds) or null.  Only the lattice kinds in mixed precision take mirror images: in the
+// with npx = 2, v[1] of its mirror image (-ihex, -i); npx = 0: a lane without a pixel, which
+// repeats one.  rv: its radial-table entry (midpoint grid, radial kinds) or null.  Only the lattice kinds in mixed precision take mirror images: in the
 // midpoint grid the peak sum at -q is the one at q (each Friedel pair swaps its two terms), and
 // so is every factor of |q|; the oriented cylinder's rod factor is evaluated at both.
 // MODE kHot: *cold reports a pixel that needs an FP64 path, with its state in *cp; kFix:
 // finishes such a pixel from *cp.
 template <int KIND, int PREC, int MODE = kFull>
-__device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* v, bool mir,
+__device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* v, int npx,
                                              unsigned long long* stats = nullptr, const Radial* rv = nullptr,
                                              bool* cold = nullptr, ColdPix* cp = nullptr) {
     const csx_scalars& s = d.s;
+    const bool mir = npx == 2;
     // The mixed FCC path with a radial entry needs only |q| and the pixel indices.
     if (!(rv && (KIND == K_FCC || KIND == K_ISO_LAT) && PREC == CSX_PREC_MIXED)) need_q(s, P3);
     const double qx = P3.qx, qy = P3.qy, qz = P3.qz;
@@ -1476,12 +1478,12 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                     else pixel_dirs(s, P3, q, L);
                     if (s.centerbeam) near_one_add<false, kPrecise>(d, W, L, L64, P3, q, width, inten);
                     else near_one_add<true, kPrecise>(d, W, L, L64, P3, q, width, inten);
-                    if (stats) atomicAdd(&stats[2], 1ull);
+                    if (stats) atomicAdd(&stats[2], (unsigned long long)npx);
                 }
             } else {
                 inten = s.centerbeam
-                            ? lattice_mixed<false, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, stats)
-                            : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, stats);
+                            ? lattice_mixed<false, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, npx, stats)
+                            : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, npx, stats);
             }
             radint = (s.iso != 0) ? iso_mixed(d, q) : 0.0;
             factors();
@@ -1519,14 +1521,14 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 if (__ballot(window)) {
                     if (window) need_q(s, P3);
                     coop_window_sum64<kPrecise>(d, W, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, window, inten);
-                    if (stats && window) atomicAdd(&stats[1], 1ull);
+                    if (stats && window) atomicAdd(&stats[1], (unsigned long long)npx);
                 }
                 want3 = want3 || (window && loose(inten, 1.0e-13));
                 inten2 = inten;
                 if (__ballot(want3)) {
                     if (want3) need_q(s, P3);
                     coop_full_sum64(d, PixArgs{P3.qx, P3.qy, P3.qz, q, width}, want3, mir, inten, inten2, radint);
-                    if (stats && want3) atomicAdd(&stats[4], 1ull);
+                    if (stats && want3) atomicAdd(&stats[4], (unsigned long long)npx);
                 }
             }
         }
@@ -1596,6 +1598,7 @@ __host__ __device__ inline Cover make_cover(int x0, int x1, int y0, int y1, int 
 struct CoverPix {
     int ihex, i;
     bool in, mir;  // the lane has a pixel of the block; its mirror image is this lane's as well
+    int npx;       // in + mir
 };
 // Lanes without a pixel repeat a neighbouring one (the mixed path needs all 64 lanes).
 __device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int w) {
@@ -1631,6 +1634,7 @@ __device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int w) {
             p.mir = p.in && row && k > 0 && k < c.x1;
         }
     }
+    p.npx = (int)p.in + (int)p.mir;
     return p;
 }
 // The kinds whose value is the same, bit for bit, at (+-qx, +-qy): the |q|-only ones; at
@@ -1739,7 +1743,7 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
     bool cold = false;
     ColdPix cpx;
     double v[2];
-    pixel_values<KIND, PREC, MODE>(d, P3, v, p.mir, stats, rv, &cold, &cpx);
+    pixel_values<KIND, PREC, MODE>(d, P3, v, p.npx, stats, rv, &cold, &cpx);
     if constexpr (MODE == kHot) {
         // queue the cold pixels (lanes without a pixel repeat one)
         const bool mine = cold && p.in;
@@ -1823,7 +1827,7 @@ k_image_lat_fix(const DevSet d, const Cover c, double* __restrict__ out, unsigne
             rv = rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
         }
         double v[2];
-        pixel_values<KIND, PREC, kFix>(d, P3, v, mir, stats, rv, nullptr, &cp);
+        pixel_values<KIND, PREC, kFix>(d, P3, v, have ? 1 + (int)mir : 0, stats, rv, nullptr, &cp);
         if (have) out[(size_t)(cp.ihex - c.x0) + W * (size_t)(cp.i - c.y0)] = v[0];
         if (mir) out[(size_t)(-cp.ihex - c.x0) + W * (size_t)(-cp.i - c.y0)] = v[1];
     }
@@ -1902,12 +1906,12 @@ struct TileSum {
 // sets array, the isotropic cylinder's P(q) came out wrong above its series radius (with and
 // without a lattice).  The sphere and z-oriented cylinder lattice kinds read them in place.
 template <int KIND, int PREC>
-__device__ __forceinline__ void set_pixel(const FitSet& f, PixQ& P3, double* v, bool mir, const Radial* rv) {
+__device__ __forceinline__ void set_pixel(const FitSet& f, PixQ& P3, double* v, int npx, const Radial* rv) {
     if constexpr (KIND == K_FCC || KIND == K_BCT) {
-        pixel_values<KIND, PREC>(f.d, P3, v, mir, nullptr, rv);
+        pixel_values<KIND, PREC>(f.d, P3, v, npx, nullptr, rv);
     } else {
         const DevSet d = f.d;
-        pixel_values<KIND, PREC>(d, P3, v, mir, nullptr, rv);
+        pixel_values<KIND, PREC>(d, P3, v, npx, nullptr, rv);
     }
 }
 
@@ -1930,7 +1934,7 @@ __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __re
             rv = f.rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
         }
         double v[2];
-        set_pixel<KIND, PREC>(f, P3, v, p.mir, rv);
+        set_pixel<KIND, PREC>(f, P3, v, p.npx, rv);
         for (int k = 0; k < 2; ++k) {
             if (!(k ? p.mir : p.in)) continue;
             const int x = (k ? -p.ihex : p.ihex) - f.cov.x0, y = (k ? -p.i : p.i) - f.cov.y0;
@@ -2029,7 +2033,7 @@ __device__ __forceinline__ void image_batch_tiles(const FitSet* __restrict__ set
         rv = f.rtab + (a <= b ? tri_index(a, b) : tri_index(b, a));
     }
     double v[2];
-    set_pixel<KIND, PREC>(f, P3, v, p.mir, rv);
+    set_pixel<KIND, PREC>(f, P3, v, p.npx, rv);
     double* out = const_cast<double*>(f.data);
     if (p.in) out[(size_t)(p.ihex - f.cov.x0) + (size_t)f.w * (size_t)(p.i - f.cov.y0)] = v[0];
     if (p.mir) out[(size_t)(-p.ihex - f.cov.x0) + (size_t)f.w * (size_t)(-p.i - f.cov.y0)] = v[1];

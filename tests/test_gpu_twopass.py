@@ -14,7 +14,7 @@ from crystalscatter_amd import SasCalc, _lib
 pytestmark = pytest.mark.gpu
 
 
-def _render_stats(p, prec):
+def _render_stats(p, prec, block=None):
     import torch
     e = SasCalc(device=0, params=p)
     e.set("ignore_cbs", 1)
@@ -22,7 +22,7 @@ def _render_stats(p, prec):
     L = _lib.lib()
     ctx = L.csx_engine_ctx(e._h)
     s = e.scalars()
-    g = _lib.Grid(s.xmin, s.xmax, s.ymin, s.ymax)
+    g = _lib.Grid(*(block or (s.xmin, s.xmax, s.ymin, s.ymax)))
     out = torch.empty((s.xmax - s.xmin) * (s.ymax - s.ymin), dtype=torch.float64, device="cuda")
     st = (ctypes.c_uint64 * 5)()
     assert L.csx_render_stats(ctx, ctypes.byref(g), {"ref64": 0, "mixed": 1}[prec], ctypes.c_void_p(out.data_ptr()),
@@ -61,6 +61,22 @@ def test_fix_pass_is_exercised():
         _, st = _render_stats(CASES[name], "mixed")
         total += st[1] + st[4] + (st[2] if name == "fcc_centre_beam" else 0)
     assert total > 0
+
+
+@pytest.mark.parametrize("z", [5, 16, 37])
+@pytest.mark.parametrize("kind", ["fcc", "bct"])
+def test_counts_are_of_pixels(kind, z):
+    """Peaks so broad that every pixel takes every pair: whether a pixel has pairs near one and
+    whether the guard takes it again does not depend on how the pixels are spread over waves, so
+    the counts of the whole image (mirror images, half-filled strips) are those of its four
+    quadrants (every pixel on its own)."""
+    p = dict(CFG3 if kind == "fcc" else manifest()["fixtures"]["cfg4_bct.npz"]["params"][0], GridPoints=z,
+             EditDomainSize=4, EditAzi=60)
+    _, st = _render_stats(p, "mixed")
+    parts = [_render_stats(p, "mixed", (x, x + z, y, y + z))[1] for x in (-z, 0) for y in (-z, 0)]
+    print(kind, z, st, parts, flush=True)
+    for k in (1, 2, 4):
+        assert st[k] == sum(q[k] for q in parts)
 
 
 def test_pass_timing_ring():
