@@ -1943,7 +1943,8 @@ __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __re
             if (!fit_masked(s, f.m, f.data, f.w, x, y)) {
                 const double dv = f.data[idx];
                 if (v[k] > 0 && dv > 0) {
-                    const double a = (log(v[k]) - log(dv)) * 0.43429448190325182765;  // log10(v / dv)
+                    // the reference's quotients: which terms come out exactly 0 is counted
+                    const double a = log(v[k]) / log(10.) - log(dv) / log(10.);
                     tk = a * a;
                 }
             }

@@ -402,3 +402,22 @@ def test_bcc_512_against_oracle_random_pixels(oracle_lib):
     assert r.max() < 1e-4
     a = img.reshape(512, 512)[1:, 1:]
     assert rel_err(a, a[::-1, ::-1]).max() < 1e-6
+
+
+@pytest.mark.parametrize("prec", ["ref64", "mixed"])
+def test_objective_counts_terms_that_are_not_zero(prec):
+    """The objective counts the terms that are not exactly 0.  Data a few roundings off the image
+    decide that by the last bits of the two quotients log(x)/log(10), here formed with the
+    device's own log (torch) and IEEE divisions."""
+    import torch
+    e, img = _calc(dict(CFG1, GridPoints=64), prec)
+    rng = np.random.default_rng(3)
+    data = img * (1 + 2.0 ** -52 * rng.integers(-8, 9, img.size))
+    v, d = (torch.from_numpy(a).cuda() for a in (img, data))
+    ten = torch.full_like(v, np.log(10.0))
+    t = (torch.log(v) / ten - torch.log(d) / ten) ** 2
+    ok = (v > 0) & (d > 0)
+    e.setFitData(128, 128, data)
+    s, cnt, nan = e.doFitCalculation(precision=prec)
+    assert nan == 0 and cnt == int((ok & (t != 0)).sum()) and 0 < cnt < img.size
+    assert s == pytest.approx(float(t[ok].sum()), rel=1e-12)
