@@ -1158,68 +1158,130 @@ __device__ double romb_delta_cyl(const DevSet& d, double qx, double qy, int i1) 
     return pq;
 }
 
+// Physics-mode orientation average: kCqWaves waves share 64 pixels, in kCqChunk polar nodes at a
+// time.  LDS: the rod factor's table, one cubic c0 + t (c1 + t (c2 + t c3)) a knot interval (one
+// 16-byte read an evaluation and no coefficient arithmetic), the node tables, the azimuth sums
+// of a chunk and the series' state; 75.9 KB, so two workgroups a CU (160 KB) and four waves a
+// SIMD.  File-scope LDS, so that every access compiles to a ds_read with a 32-bit offset.
+constexpr int kCqWaves = 8, kCqChunk = 32;
+struct CgState {  // small-q series of a pixel: its sum, and whether it has yet to converge
+    double sum;
+    int left;
+};
+__shared__ float4 g_cq_tab[kCqTab];
+__shared__ float4 g_cq_dl[kCqDelta];
+__shared__ float g_cq_tt[kCqPsi / 2];
+__shared__ float g_cq_sk[kCqChunk][64];
+__shared__ CgState g_cq_series[64];
+
 // Small-q double series of the Gaussian orientation average (formpq_partCylinder ordis 0,
 // Source/sc_lib_formpq_partCylinder.h:133-203), orientation cases 1..3:
 //   pql = 1 + sum_n c1p[n] sum_m c11pm[n-m][m] X^m Y^(n-m)
 // with (X, Y) = (qxs^2, qys^2), swapped for case 3.  The inner sum is evaluated by Horner in
 // the ratio of the smaller to the larger of X and Y (no power tables; the reference builds
 // X^m and Y^(n-m) as running products, so the two agree to rounding).
-// Wave-cooperative (called by all 64 lanes; `want` per lane): the requesting lanes are taken one
-// at a time (of nparts waves with the same pixels, this one takes every nparts-th request), and
-// lane j forms the inner sum and powers of order n = j + 1 (then j + 65); the terms are added in
-// order.  One lane on its own walks up
-// to 120 x 120 / 2 dependent loads where the series does not converge: 0.2 ms, longer than the
-// rest of a 512^2 pattern.
-__device__ double cyl_gauss_series(const DevSet& d, double qxs, double qys, int oc, bool want, int part, int nparts) {
+// Called by all 64 lanes; `want` per lane.  Most pixels converge within a few orders, so the first
+// kCgFirst are taken for all of them at once: each lane for its own pixel in turn, or, where the
+// kCqWaves waves of a workgroup hold the same pixels (SHARED), eight lanes of wave `part` for one
+// of its eight, lane j the orders j + 1 and j + 9.  The pixels left over are then taken one at a
+// time (SHARED: the waves take turns), lane j forming the inner sum and powers of order n = j + 1
+// (then j + 65): one lane on its own walks up to 120 x 120 / 2 dependent loads where the series
+// does not converge.  The terms are added in order everywhere.  A 512^2 pattern of the series alone:
+// 11 us (385 us, in FP64 1146, with all orders of one pixel at a time); one that leaves it at two
+// fifths of qmax: 328 us (902 us each lane for itself to the end).
+constexpr int kCgFirst = 16;
+static_assert(kCqWaves * 8 == 64, "eight pixels a wave");
+template <bool SHARED>
+__device__ double cyl_gauss_series(const DevSet& d, double qx, double qy, int oc, bool want, int part) {
     const double* c1p = carr_of<0>(d);
     const double* c11 = d.carr11pm;  // [n][m], CSX_NIM2 columns
-    const int lane = (int)threadIdx.x & 63;
-    unsigned long long todo = __ballot(want);
-    double mine = 1.0;
+    const int lane = (int)threadIdx.x & 63, sub = lane & 7;
+    const int own = SHARED ? 8 * part + (lane >> 3) : lane;
+    struct Arg {
+        double big, r;  // r = small/large <= 1, the Horner variable
+        bool xs;
+    };
+    auto arg_of = [&](double px, double py) {
+        const double X = (oc == 3) ? py * py : px * px, Y = (oc == 3) ? px * px : py * py;
+        Arg a;
+        a.xs = X <= Y;
+        a.big = a.xs ? Y : X;
+        a.r = a.xs ? (Y > 0 ? X / Y : 0.0) : (X > 0 ? Y / X : 0.0);
+        return a;
+    };
+    // c1p[n] sum_m c11[n-m][m] X^m Y^(n-m) = c1p[n] big^n sum_k a_k r^k, with k = m (X small) or n-m
+    auto term_of = [&](const Arg& g, int n) {
+        double bn = g.big;
+        double h = g.xs ? c11[0 * CSX_NIM2 + n] : c11[n * CSX_NIM2 + 0];
+#pragma unroll 4
+        for (int k = n - 1; k >= 0; --k) {
+            const double a = g.xs ? c11[(n - k) * CSX_NIM2 + k] : c11[k * CSX_NIM2 + (n - k)];
+            h = h * g.r + a;
+            if (k > 0) bn *= g.big;
+        }
+        return c1p[n] * (h * bn);
+    };
+    const Arg mine = arg_of(SHARED ? __shfl(qx, own, 64) : qx, SHARED ? __shfl(qy, own, 64) : qy);
+    double pql = 1.0, old = 0.0;
+    bool go = (__ballot(want) >> own) & 1ull;
+    for (int n = 1; n <= kCgFirst && __ballot(go); n += SHARED ? 8 : 1) {
+        if constexpr (SHARED) {
+            const double term = term_of(mine, n + sub);
+            double at = 0.0, before = 0.0, sum = pql, last = old;
+            for (int j = 0; j < 8; ++j) {  // the sums up to each order; lane j keeps its own two
+                sum += __shfl(term, (lane & 56) + j, 64);
+                if (j == sub) {
+                    at = sum;
+                    before = last;
+                }
+                last = sum;
+            }
+            const unsigned done = (unsigned)(__ballot(fabs((at - before) / at) < 0.0001) >> (lane & 56)) & 255u;
+            const double end = __shfl(at, (lane & 56) + (done ? __builtin_ctz(done) : 7), 64);
+            if (go) {
+                pql = old = end;
+                go = !done;
+            }
+        } else if (go) {
+            pql += term_of(mine, n);
+            go = !(fabs((pql - old) / pql) < 0.0001);
+            old = pql;
+        }
+    }
+    if constexpr (SHARED) {
+        if (sub == 0) g_cq_series[own] = CgState{pql, go};
+        __syncthreads();
+        pql = g_cq_series[lane].sum;  // by pixel from here on
+        go = g_cq_series[lane].left;
+        if (!__ballot(go)) return pql;
+        __syncthreads();
+    }
+    unsigned long long todo = __ballot(go);
     for (int i = 0; todo; ++i) {
         const int l = __builtin_ctzll(todo);
         todo &= todo - 1;
-        if (i % nparts != part) continue;
-        const double px = __shfl(qxs, l, 64), py = __shfl(qys, l, 64);
-        const double X = (oc == 3) ? py * py : px * px, Y = (oc == 3) ? px * px : py * py;
-        const bool xs = X <= Y;            // Horner variable r = small/large <= 1
-        const double big = xs ? Y : X, r = xs ? (Y > 0 ? X / Y : 0.0) : (X > 0 ? Y / X : 0.0);
-        double pql = 1.0, old = 0.0;
-        bool go = true;
-        for (int base = 0; go && base < 120; base += 64) {
-            const int n = min(base + 1 + lane, 120);
-            // sum_m c11[n-m][m] X^m Y^(n-m) = big^n * sum_k a_k r^k, with k = m (X small) or n-m
-            double bn = big;
-            double h = xs ? c11[0 * CSX_NIM2 + n] : c11[n * CSX_NIM2 + 0];
-#pragma unroll 4
-            for (int k = n - 1; k >= 0; --k) {
-                const double a = xs ? c11[(n - k) * CSX_NIM2 + k] : c11[k * CSX_NIM2 + (n - k)];
-                h = h * r + a;
-                if (k > 0) bn *= big;
-            }
-            const double term = c1p[n] * (h * bn);
-            for (int j = 0; go && j < min(64, 120 - base); ++j) {
-                pql += __shfl(term, j, 64);
-                go = !(fabs((pql - old) / pql) < 0.0001);
-                old = pql;
+        if (SHARED && i % kCqWaves != part) continue;
+        const Arg g = arg_of(__shfl(qx, l, 64), __shfl(qy, l, 64));
+        double sum = 1.0, last = 0.0;
+        bool more = true;
+        for (int base = 0; more && base < 120; base += 64) {
+            const double term = term_of(g, min(base + 1 + lane, 120));
+            for (int j = 0; more && j < min(64, 120 - base); ++j) {
+                sum += __shfl(term, j, 64);
+                more = !(fabs((sum - last) / sum) < 0.0001);
+                last = sum;
             }
         }
-        if (lane == l) mine = pql;
+        if (lane != l) continue;
+        if constexpr (SHARED) g_cq_series[l].sum = sum;
+        else pql = sum;
     }
-    return mine;
+    if constexpr (SHARED) {
+        __syncthreads();
+        pql = g_cq_series[lane].sum;
+    }
+    return pql;
 }
-
-// Physics-mode orientation average: kCqWaves waves share 64 pixels, in kCqChunk polar nodes at a
-// time.  LDS: the rod factor's table, one cubic c0 + t (c1 + t (c2 + t c3)) a knot interval (one
-// 16-byte read an evaluation and no coefficient arithmetic), the node tables, the azimuth sums
-// of a chunk and the series' results; 75.4 KB, so two workgroups a CU (160 KB) and four waves a
-// SIMD.  File-scope LDS, so that every access compiles to a ds_read with a 32-bit offset.
-constexpr int kCqWaves = 8, kCqChunk = 32;
-__shared__ float4 g_cq_tab[kCqTab];
-__shared__ float4 g_cq_dl[kCqDelta];
-__shared__ float g_cq_tt[kCqPsi / 2];
-__shared__ float g_cq_sk[kCqChunk][64];
-__shared__ double g_cq_series[64];
 
 __device__ __forceinline__ void cq_fill(const DevSet& d) {
     for (int k = threadIdx.x; k < kCqTab; k += kCqWaves * 64) {
@@ -1343,7 +1405,10 @@ __device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, d
             if constexpr (KIND == K_CYL_GAUSS_Q) {
                 // physics mode: oc in 1..3, tables in LDS.  The workgroup's waves hold the same
                 // 64 pixels and share the nodes.
-                if (__ballot(!series)) pql = cyl_gauss_quad(d, qa, qb, oc);
+                if (__ballot(!series)) {
+                    cq_fill(d);
+                    pql = cyl_gauss_quad(d, qa, qb, oc);
+                }
             } else if (!series) {
                 // the reference's nested Romberg; in reference mode the general case (oc = 0)
                 // has an identically zero integrand
@@ -1351,18 +1416,9 @@ __device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, d
             }
             if (__ballot(series)) {
                 const bool want = series && oc >= 1 && oc <= 3;
-                double v;
-                if constexpr (KIND == K_CYL_GAUSS_Q) {
-                    const int wave = uniform_i((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
-                    const double part = cyl_gauss_series(d, qa, qb, oc, want, wave, kCqWaves);
-                    const unsigned long long req = __ballot(want);
-                    const int place = __popcll(req & ((1ull << lane) - 1));  // of this lane's request
-                    if (want && place % kCqWaves == wave) g_cq_series[lane] = part;
-                    __syncthreads();
-                    v = want ? g_cq_series[lane] : 1.0;
-                } else {
-                    v = cyl_gauss_series(d, qa, qb, oc, want, 0, 1);
-                }
+                constexpr bool kShared = KIND == K_CYL_GAUSS_Q;
+                const int part = kShared ? uniform_i((int)threadIdx.x >> 6) : 0;
+                const double v = cyl_gauss_series<kShared>(d, qa, qb, oc, want, part);
                 if (series) pql = want ? v : 1.0;
             }
         }
@@ -1637,14 +1693,25 @@ __device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int w) {
     p.npx = (int)p.in + (int)p.mir;
     return p;
 }
+// Whether a block of the midpoint grid lies below the limit of the Gaussian cylinders' small-q
+// series, the corner's |q| with a margin above any rounding of it.
+inline bool inside_series(const csx_scalars& s, int x0, int x1, int y0, int y1) {
+    if (s.centerbeam || s.use1d) return false;
+    const double h = std::max(std::abs((double)x0), std::abs((double)x1 - 1));
+    const double i = std::max(std::abs((double)y0), std::abs((double)y1 - 1));
+    return std::hypot(h, i) * std::abs(s.qmax) / s.zmax * (1 + 1e-12) + 2e-9 < 0.4 * s.limq[0];
+}
 // The kinds whose value is the same, bit for bit, at (+-qx, +-qy): the |q|-only ones; at
 // (qx, +-qy): the physics-mode orientation average about a direction in the x-z plane (phi is 0
 // in the general case) -- its argument along the axis carries +1e-10, so it is not even in qx.
 // A 128^2 sphere pattern: 28 us with a radial table before the image, 5 us without.
+// The small-q series of the same kind is one of squares: a grid that it alone covers is even in both.
 inline int even_cover(const DevSet& d, int kind, int x0, int x1, int y0, int y1) {
     if (d.s.centerbeam || d.s.use1d || x1 <= 0 || y1 <= 0 || x0 != -x1 || y0 != -y1) return kPlain;
     if (kind == K_SPHERE || kind == K_CUBE || kind == K_CYL_ISO) return kQuarter;
     if (kind == K_CYL_GAUSS_Q && (d.s.orcase == 1 || (d.s.orcase == 0 && d.s.sinphic == 0.0))) return kHalf;
+    if (kind == K_CYL_GAUSS && inside_series(d.s, x0, x1, y0, y1) && (d.s.orcase != 0 || d.s.sinphic == 0.0))
+        return kQuarter;
     return kPlain;
 }
 // Mirror images serve the lattice kinds' Gaussian peak sums in mixed precision, in the
@@ -1733,7 +1800,6 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
     // (Gaussian cylinders, quadrature: every wave of the workgroup holds quadrant blockIdx.z)
     const CoverPix p = cover_pixel(c, t, KIND == K_CYL_GAUSS_Q ? (int)blockIdx.z : (int)threadIdx.x >> 6);
     PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
-    if constexpr (KIND == K_CYL_GAUSS_Q) cq_fill(d);
     if (!__ballot(p.in)) return;
     const Radial* rv = nullptr;
     if (rtab) {
@@ -3107,11 +3173,15 @@ static int put_table(csx_ctx* c, DevBuf& b, const std::vector<T>& v) {
     return CSX_OK;
 }
 
-// Kernel kind of a render: the key's kind, or the physics-mode quadrature kernel for
-// Gaussian cylinders in mixed precision.
-static int render_kind(const csx_ctx* c, int precision) {
-    const int k = kind_of(c->set.s.combo_key);
-    if (k == K_CYL_GAUSS && c->set.s.fix_orcase && precision == CSX_PREC_MIXED && c->set.cq_tab) return K_CYL_GAUSS_Q;
+// Kernel kind of a render: the key's kind, or the physics-mode quadrature kernel for Gaussian
+// cylinders in mixed precision, unless no pixel takes the quadrature: its workgroups of eight waves
+// on 64 pixels serve the series badly (512^2: 20 us for the other kernel's 11).
+static int render_kind(const csx_ctx* c, int precision, const csx_grid& g) {
+    const csx_scalars& s = c->set.s;
+    const int k = kind_of(s.combo_key);
+    if (k == K_CYL_GAUSS && s.fix_orcase && precision == CSX_PREC_MIXED && c->set.cq_tab &&
+        !inside_series(s, g.xmin, g.xmax, g.ymin, g.ymax))
+        return K_CYL_GAUSS_Q;
     return k;
 }
 
@@ -3468,7 +3538,7 @@ int csx_render(csx_ctx* c, const csx_grid* g, int precision, double* d_out) {
     if (g->xmax <= g->xmin || g->ymax <= g->ymin) return fail(c, CSX_E_ARG, "empty grid");
     if (precision != CSX_PREC_REF64 && precision != CSX_PREC_MIXED) return fail(c, CSX_E_ARG, "bad precision");
     HIPCHK(c, hipSetDevice(c->device));
-    const int kind = render_kind(c, precision);
+    const int kind = render_kind(c, precision, *g);
     if (c->timing) HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     if (int rc = render_launch(c, kind, precision, *g, d_out, nullptr)) return rc;
     if (c->timing) {
@@ -3488,7 +3558,7 @@ int csx_render_stats(csx_ctx* c, const csx_grid* g, int precision, double* d_out
     HIPCHK(c, c->stats.ensure(CSX_NSTATS * sizeof(uint64_t)));
     const std::vector<uint64_t> zero(CSX_NSTATS, 0);
     HIPCHK(c, hipMemcpyAsync(c->stats.p, zero.data(), CSX_NSTATS * sizeof(uint64_t), hipMemcpyHostToDevice, c->stream));
-    const int kind = render_kind(c, precision);
+    const int kind = render_kind(c, precision, *g);
     if (int rc = render_launch(c, kind, precision, *g, d_out, (unsigned long long*)c->stats.p)) return rc;
     HIPCHK(c, hipMemcpyAsync(h_stats, c->stats.p, CSX_NSTATS * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
