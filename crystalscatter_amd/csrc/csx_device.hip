@@ -3068,7 +3068,7 @@ TileSum* scratch_address(int device) {
 // Radial pre-pass for kinds whose form factors depend on |q| only, in the midpoint grid.
 template <int K, int P>
 static void launch_radial(const DevSet& d, const csx_grid& g, Radial* rtab, hipStream_t st) {
-    if constexpr (radial_kind(K)) {
+    if constexpr (radial_kind(K) && K != K_CUBE) {  // (cubes: batches only)
         const int m = std::max(std::max(std::abs(g.xmin), std::abs(g.xmax - 1)),
                                std::max(std::abs(g.ymin), std::abs(g.ymax - 1)));
         const int total = (m + 1) * (m + 2) / 2;
@@ -3185,17 +3185,31 @@ static int render_kind(const csx_ctx* c, int precision, const csx_grid& g) {
     return k;
 }
 
-// Radial table of a render (midpoint grid, radial lattice kinds), sized for the grid, and its
-// slot; null otherwise.  The |q|-only kinds without a lattice evaluate each pixel of the quarter
-// cover instead: twice the table's evaluations, but one launch and no events (isotropic spheres
-// at 128^2 took 26 us, most of it the second launch and the stream hand-over; 1024^2 the same).
-static int radial_table(csx_ctx* c, const csx_grid& g, Radial** out, int* slot) {
+// Whether a pattern of |q| alone without a lattice takes the table: its pixels cost little more than
+// the table's entries, and the second launch with its stream hand-over costs about 20 us.  Spheres
+// and cylinders do on a plain cover (a block of a detector, a quadrant, a half) where the table saves
+// enough evaluations; on the quarter cover, with at most twice the table's, and for cubes (half a
+// sphere's cost) it never wins.  Back to back, us with /
+// without it:
+//   spheres    half 512 25/20, 700 28/32, 1024 40/69;  quadrant 1024 38/36, 1448 59/62, 2048 103/124
+//   cylinders  half 700 29/27, 1024 38/55, 2048 108/187;  quadrant 1448 60/51, 2048 100/97
+//   cubes      half 1024 39/33, 2048 107/109;  quadrant 2048 93/58
+static bool table_pays(int kind, const Cover& cov, long long entries) {
+    if (cov.mode != kPlain || (kind != K_SPHERE && kind != K_CYL_ISO)) return false;
+    const long long px = (long long)(cov.x1 - cov.x0) * (cov.y1 - cov.y0);
+    return px - entries >= 700000 && (kind == K_SPHERE || px >= 3 * entries);
+}
+// Radial table of a render (midpoint grid, radial kinds; without a lattice where table_pays), sized
+// for the grid, and its slot; null otherwise.
+static int radial_table(csx_ctx* c, const Cover& g, Radial** out, int* slot) {
     *out = nullptr;
     *slot = -1;
-    if (!radial_kind(kind_of(c->set.s.combo_key)) || !lattice_kind(kind_of(c->set.s.combo_key)) || c->set.s.centerbeam || c->set.s.use1d) return CSX_OK;
-    const long long m = std::max(std::max(std::llabs(g.xmin), std::llabs((long long)g.xmax - 1)),
-                                 std::max(std::llabs(g.ymin), std::llabs((long long)g.ymax - 1)));
+    const int kind = kind_of(c->set.s.combo_key);
+    if (!radial_kind(kind) || c->set.s.centerbeam || c->set.s.use1d) return CSX_OK;
+    const long long m = std::max(std::max(std::llabs(g.x0), std::llabs((long long)g.x1 - 1)),
+                                 std::max(std::llabs(g.y0), std::llabs((long long)g.y1 - 1)));
     if (m > 46000) return CSX_OK;  // triangle index would overflow int: evaluate per pixel
+    if (!lattice_kind(kind) && !table_pays(kind, g, (m + 1) * (m + 2) / 2)) return CSX_OK;
     const int sl = c->rslot;
     const size_t bytes = (size_t)((m + 1) * (m + 2) / 2) * sizeof(Radial);
     if (c->radial[sl].n < bytes) {
@@ -3244,9 +3258,13 @@ static int radial_table(csx_ctx* c, const csx_grid& g, Radial** out, int* slot) 
 // Back-to-back renders thus overlap a pre-pass with the previous image kernel.
 static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g, double* out,
                          unsigned long long* stats) {
+    const int mode = mirror_set(c->set, kind, precision, g.xmin, g.xmax, g.ymin, g.ymax)
+                         ? kMirror
+                         : even_cover(c->set, kind, g.xmin, g.xmax, g.ymin, g.ymax);
+    const Cover cov = make_cover(g.xmin, g.xmax, g.ymin, g.ymax, mode);
     Radial* rtab = nullptr;
     int sl = -1;
-    if (int rc = radial_table(c, g, &rtab, &sl)) return rc;
+    if (int rc = radial_table(c, cov, &rtab, &sl)) return rc;
     if (rtab) {
         if (c->img_recorded[sl]) HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_img[sl], 0));
         DISPATCH_KIND(kind, precision, launch_radial, c->set, g, rtab, c->side);
@@ -3254,10 +3272,6 @@ static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g,
         HIPCHK(c, hipEventRecord(c->ev_rad[sl], c->side));
         HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_rad[sl], 0));
     }
-    const int mode = mirror_set(c->set, kind, precision, g.xmin, g.xmax, g.ymin, g.ymax)
-                         ? kMirror
-                         : even_cover(c->set, kind, g.xmin, g.xmax, g.ymin, g.ymax);
-    const Cover cov = make_cover(g.xmin, g.xmax, g.ymin, g.ymax, mode);
     // Lattice kinds in mixed precision render in two passes (hot, then fix over a queue of at
     // most one slot per wave), unless unpaired reflections send every pixel to FP64.
     ColdQueue cq{};
