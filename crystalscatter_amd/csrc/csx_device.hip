@@ -718,7 +718,7 @@ struct ColdPix {
     int ihex, i;
     double inten, dropped;
     int b0, b1, band0, band1;
-    int flags;  // 1: near-one pairs in the window, 2: unpaired reflections, 4: placeholder lane
+    int flags;  // 1: near-one pairs in the window, 4: placeholder lane, 8: its mirror image as well
     int pad;
 };
 
@@ -733,10 +733,11 @@ struct ColdQueue {
 };
 
 // How a pixel is evaluated.  kFull: every path in one pass.  kHot: the common paths only;
-// a pixel that needs an FP64 path (near-one pairs, the conditioning guard, unpaired
-// reflections) is reported `cold` and its whole wave is evaluated again by kFix, which runs
-// every path and does not repeat the pair-evaluation counts.
-enum PixMode { kFull = 0, kHot = 1, kFix = 2 };
+// a pixel that needs an FP64 path (near-one pairs, the conditioning guard) is reported `cold`
+// and finished by kFix, which runs every path and does not repeat the pair-evaluation counts.
+// kSolo: one pass over a set with unpaired reflections (no mirror images, every pixel by the
+// full sum).
+enum PixMode { kFull = 0, kHot = 1, kFix = 2, kSolo = 3 };
 
 // Adds to inten, band by band, the FP64 terms (the reference's formula) of the window's pairs
 // with |q^.u| > kNearOne, which the pair loop left out: L (FP32 loop) or L64 (precise loop)
@@ -758,11 +759,11 @@ __device__ __forceinline__ void near_one_add(const DevSet& d, const Window& W, c
 // Mixed-precision anisotropic peak sum (sum over reflections of sq*mhkl*fhkl*psi).  Must be
 // called by all 64 lanes of a wave: the wave's union of per-lane windows selects the pairs.
 // Pairs outside the window, and second Friedel terms where they cannot reach 2^cut, are
-// dropped: every dropped term is below 2^cut * A.  need_exact: unpaired reflections exist.
+// dropped: every dropped term is below 2^cut * A.
 // npx: the pixels that the lane's value serves (for the counts).
 template <bool PLANAR, bool PRECISE, int MODE = kFull>
-__device__ __forceinline__ double lattice_mixed(const DevSet& d, PixQ& P3, double q, double width, bool& need_exact,
-                                double& dropped, Window& W, int npx, unsigned long long* stats) {
+__device__ __forceinline__ double lattice_mixed(const DevSet& d, PixQ& P3, double q, double width, double& dropped,
+                                                Window& W, int npx, unsigned long long* stats) {
     const csx_scalars& s = d.s;
     PixelConsts L;
     pixel_dirs(s, P3, q, L);
@@ -901,7 +902,6 @@ __device__ __forceinline__ double lattice_mixed(const DevSet& d, PixQ& P3, doubl
         atomicAdd(&stats[3], (unsigned long long)(any_two ? 1 : 0));
     }
     if (MODE != kFix && stats && flag) atomicAdd(&stats[2], (unsigned long long)npx);
-    need_exact = d.nsingle > 0;
     return inten;
 }
 
@@ -1440,7 +1440,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                                              unsigned long long* stats = nullptr, const Radial* rv = nullptr,
                                              bool* cold = nullptr, ColdPix* cp = nullptr) {
     const csx_scalars& s = d.s;
-    const bool mir = npx == 2;
+    const bool mir = MODE != kSolo && npx == 2;
     // The mixed FCC path with a radial entry needs only |q| and the pixel indices.
     if (!(rv && (KIND == K_FCC || KIND == K_ISO_LAT) && PREC == CSX_PREC_MIXED)) need_q(s, P3);
     const double qx = P3.qx, qy = P3.qy, qz = P3.qz;
@@ -1450,7 +1450,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
     } else {
         // P(q) and <F>^2 at the pixel (0) and, for the oriented cylinder with NV = 2, at its
         // mirror image (1)
-        constexpr int NV = KIND == K_BCT && PREC == CSX_PREC_MIXED ? 2 : 1;
+        constexpr int NV = KIND == K_BCT && PREC == CSX_PREC_MIXED && MODE != kSolo ? 2 : 1;
         double pq[NV], fqpq[NV];
         auto factors = [&]() {
             double fq[NV];
@@ -1526,7 +1526,6 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 // one queue slot holds the cold pixels of one hot wave: the same window
                 W = Window{uniform_i(cp->b0), uniform_i(cp->b1), uniform_i(cp->band0), uniform_i(cp->band1),
                            (cp->flags & 1) != 0};
-                need_exact = (cp->flags & 2) != 0;
                 if (W.near && !(cp->flags & 4)) {
                     PixelConsts L;
                     PixelConsts64 L64;
@@ -1536,12 +1535,16 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                     else near_one_add<true, kPrecise>(d, W, L, L64, P3, q, width, inten);
                     if (stats) atomicAdd(&stats[2], (unsigned long long)npx);
                 }
+            } else if (MODE == kSolo || (MODE == kFull && d.nsingle > 0)) {
+                // unpaired reflections: every pixel takes the full sum, which needs no window
+                need_exact = true;
+                inten = 0.0;
+                W = Window{0, 0, 0, 0, false};
             } else {
-                inten = s.centerbeam
-                            ? lattice_mixed<false, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, npx, stats)
-                            : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, need_exact, dropped, W, npx, stats);
+                inten = s.centerbeam ? lattice_mixed<false, kPrecise, MODE>(d, P3, q, width, dropped, W, npx, stats)
+                                     : lattice_mixed<true, kPrecise, MODE>(d, P3, q, width, dropped, W, npx, stats);
             }
-            radint = (s.iso != 0) ? iso_mixed(d, q) : 0.0;
+            radint = (s.iso != 0 && !need_exact) ? iso_mixed(d, q) : 0.0;
             factors();
             // Conditioning guard.  szq = 1 + B - (fq/pq)*dwe with B = (fq/pq)*(2*pi*I/V)*dwe.
             // The peak sum I carries up to kRelErrFP32 (FP32 loop) or kRelErrPrecise (precise
@@ -1566,9 +1569,9 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
             const bool live = MODE != kFix || !(cp->flags & 4);
             const bool want2 = live && !need_exact && loose(inten, kPrecise ? kRelErrPrecise : kRelErrFP32);
             if constexpr (MODE == kHot) {
-                *cold = W.near || need_exact || want2;
+                *cold = W.near || want2;
                 *cp = ColdPix{P3.ihex, P3.i, inten, dropped, W.b0, W.b1, W.band0, W.band1,
-                              (W.near ? 1 : 0) | (need_exact ? 2 : 0) | (mir ? 8 : 0), 0};
+                              (W.near ? 1 : 0) | (mir ? 8 : 0), 0};
                 inten2 = inten;
             } else {
                 // straight to the full sum where the dropped mass alone is too coarse
@@ -1830,7 +1833,7 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
     const size_t W = (size_t)(c.x1 - c.x0);
     if (p.in) out[(size_t)(p.ihex - c.x0) + W * (size_t)(p.i - c.y0)] = v[0];
     if constexpr (lattice_kind(KIND)) {
-        if (p.mir) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[1];
+        if (MODE != kSolo && p.mir) out[(size_t)(-p.ihex - c.x0) + W * (size_t)(-p.i - c.y0)] = v[1];
     } else if (c.mode != kPlain && p.in) {
         // ihex (quarter: and i) <= 0; the images on the axes coincide, those of the first column
         // and row lie outside the block
@@ -1849,15 +1852,14 @@ __global__ void __launch_bounds__(image_block(KIND)) k_image(const DevSet d, con
     image_tile<KIND, PREC>(d, c, out, stats, rtab);
 }
 
-// Lattice kinds in one pass (sets with unpaired reflections, where every pixel takes an FP64
-// path): the rarely taken wave-cooperative FP64 re-sums would otherwise set the register
-// budget of the whole kernel (about 140 VGPRs, 3 waves per SIMD); capped at 128 (4 waves per
-// SIMD), only those cold paths spill.
+// Lattice kinds in one pass: FP64, and in mixed precision the sets with unpaired reflections, where
+// every pixel takes the wave-cooperative full sum (HKLmax 5, 1024^2: 5.29 ms; 5.47 with a pair
+// sum before it that nothing uses).  Capped at 128 VGPRs (4 waves per SIMD).
 template <int KIND, int PREC>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_image_lat(const DevSet d, const Cover c, double* __restrict__ out, unsigned long long* __restrict__ stats,
             const Radial* __restrict__ rtab) {
-    image_tile<KIND, PREC>(d, c, out, stats, rtab);
+    image_tile<KIND, PREC, kSolo>(d, c, out, stats, rtab);
 }
 
 // Lattice kinds, two passes.  The hot pass carries no FP64 re-sum code (no spills, more waves

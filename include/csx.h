@@ -157,7 +157,8 @@ int csx_render(csx_ctx* ctx, const csx_grid* grid, int precision, double* d_out)
  * h_stats[0] pair evaluations (lanes x pairs iterated, mixed path), [1] pixels whose peak sum
  * the conditioning guard re-took in FP64 over the window, [2] pixels with FP64 terms for
  * |q^.u| near 1, [3] waves that evaluated both Friedel terms, [4] pixels re-summed in FP64
- * over the full reflection list. */
+ * over the full reflection list (every pixel of a set with unpaired reflections, which
+ * evaluates no pair). */
 #define CSX_NSTATS 5
 int csx_render_stats(csx_ctx* ctx, const csx_grid* grid, int precision, double* d_out, uint64_t* h_stats);
 

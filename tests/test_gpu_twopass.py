@@ -79,6 +79,17 @@ def test_counts_are_of_pixels(kind, z):
         assert st[k] == sum(q[k] for q in parts)
 
 
+@pytest.mark.parametrize("z", [5, 16])
+def test_unpaired_reflections_take_the_full_sum(z):
+    """A set with unpaired reflections evaluates no pair: each pixel is summed in full, once."""
+    p = dict(manifest()["fixtures"]["cfg4_bct.npz"]["params"][0], LType=1, GridPoints=z)
+    mixed, st = _render_stats(p, "mixed")
+    ref, _ = _render_stats(p, "ref64")
+    ok = np.isfinite(ref) & (ref != 0)
+    assert st == [0, 0, 0, 0, 4 * z * z]
+    assert np.array_equal(np.isfinite(mixed), np.isfinite(ref)) and rel_err(mixed[ok], ref[ok]).max() <= 1e-4
+
+
 def test_pass_timing_ring():
     import torch
     e = SasCalc(device=0, params=dict(CFG3, GridPoints=64))
