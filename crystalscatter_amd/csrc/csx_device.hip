@@ -1975,6 +1975,7 @@ struct TileSum {
 // without a lattice).  The sphere and z-oriented cylinder lattice kinds read them in place.
 template <int KIND, int PREC>
 __device__ __forceinline__ void set_pixel(const FitSet& f, PixQ& P3, double* v, int npx, const Radial* rv) {
+    static_assert(KIND != K_CYL_GAUSS_Q, "its waves share their pixels and its tables are in LDS");
     if constexpr (KIND == K_FCC || KIND == K_BCT) {
         pixel_values<KIND, PREC>(f.d, P3, v, npx, nullptr, rv);
     } else {
@@ -3226,13 +3227,13 @@ static int radial_table(csx_ctx* c, const Cover& g, Radial** out, int* slot) {
     return CSX_OK;
 }
 
+// (K_CYL_GAUSS_Q, whose kernel has its own workgroups, is a render's alone: render_launch.)
 #define DISPATCH_KIND(kind, prec, FN, ...)                                          \
     switch (kind) {                                                                 \
     case K_SPHERE: if (prec) FN<K_SPHERE, 1>(__VA_ARGS__); else FN<K_SPHERE, 0>(__VA_ARGS__); break; \
     case K_FCC: if (prec) FN<K_FCC, 1>(__VA_ARGS__); else FN<K_FCC, 0>(__VA_ARGS__); break; \
     case K_CYL_GAUSS: if (prec) FN<K_CYL_GAUSS, 1>(__VA_ARGS__); else FN<K_CYL_GAUSS, 0>(__VA_ARGS__); break; \
     case K_CYL_ZDIR: if (prec) FN<K_CYL_ZDIR, 1>(__VA_ARGS__); else FN<K_CYL_ZDIR, 0>(__VA_ARGS__); break; \
-    case K_CYL_GAUSS_Q: FN<K_CYL_GAUSS_Q, 1>(__VA_ARGS__); break; \
     case K_CUBE: if (prec) FN<K_CUBE, 1>(__VA_ARGS__); else FN<K_CUBE, 0>(__VA_ARGS__); break; \
     case K_CYL_ISO: if (prec) FN<K_CYL_ISO, 1>(__VA_ARGS__); else FN<K_CYL_ISO, 0>(__VA_ARGS__); break; \
     case K_CUBE_ZDIR: if (prec) FN<K_CUBE_ZDIR, 1>(__VA_ARGS__); else FN<K_CUBE_ZDIR, 0>(__VA_ARGS__); break; \
@@ -3247,7 +3248,6 @@ static int radial_table(csx_ctx* c, const Cover& g, Radial** out, int* slot) {
     case K_FCC: out = (prec) ? FN<K_FCC, 1>(__VA_ARGS__) : FN<K_FCC, 0>(__VA_ARGS__); break; \
     case K_CYL_GAUSS: out = (prec) ? FN<K_CYL_GAUSS, 1>(__VA_ARGS__) : FN<K_CYL_GAUSS, 0>(__VA_ARGS__); break; \
     case K_CYL_ZDIR: out = (prec) ? FN<K_CYL_ZDIR, 1>(__VA_ARGS__) : FN<K_CYL_ZDIR, 0>(__VA_ARGS__); break; \
-    case K_CYL_GAUSS_Q: out = FN<K_CYL_GAUSS_Q, 1>(__VA_ARGS__); break; \
     case K_CUBE: out = (prec) ? FN<K_CUBE, 1>(__VA_ARGS__) : FN<K_CUBE, 0>(__VA_ARGS__); break; \
     case K_CYL_ISO: out = (prec) ? FN<K_CYL_ISO, 1>(__VA_ARGS__) : FN<K_CYL_ISO, 0>(__VA_ARGS__); break; \
     case K_CUBE_ZDIR: out = (prec) ? FN<K_CUBE_ZDIR, 1>(__VA_ARGS__) : FN<K_CUBE_ZDIR, 0>(__VA_ARGS__); break; \
@@ -3301,7 +3301,11 @@ static int render_launch(csx_ctx* c, int kind, int precision, const csx_grid& g,
         ev = e;
         ++c->pass_n;
     }
-    DISPATCH_KIND(kind, precision, launch_image, c->set, cov, out, stats, rtab, cqp, ev, c->stream);
+    if (kind == K_CYL_GAUSS_Q) {
+        launch_image<K_CYL_GAUSS_Q, CSX_PREC_MIXED>(c->set, cov, out, stats, rtab, cqp, ev, c->stream);
+    } else {
+        DISPATCH_KIND(kind, precision, launch_image, c->set, cov, out, stats, rtab, cqp, ev, c->stream);
+    }
     HIPCHK(c, hipGetLastError());
     if (rtab) {
         HIPCHK(c, hipEventRecord(c->ev_img[sl], c->stream));
