@@ -1660,14 +1660,15 @@ struct CoverPix {
     int npx;       // in + mir
 };
 // Lanes without a pixel repeat a neighbouring one (the mixed path needs all 64 lanes).
-__device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int w) {
+// (tx, ty): the workgroup's tile, t % tiles_x and t / tiles_x.
+__device__ __forceinline__ CoverPix cover_pixel(const Cover& c, int t, int tx, int ty, int w) {
     CoverPix p;
     if (t < c.main) {
         int px, py;
         tile_pixel(w, px, py);
         const int ylim = c.mode == kMirror || c.mode == kQuarter ? 0 : c.y1;
         const int xlim = c.mode == kQuarter || c.mode == kHalf ? 0 : c.x1;
-        const int ihex = c.x0 + t % c.tiles_x * kTile + px, i = c.y0 + t / c.tiles_x * kTile + py;
+        const int ihex = c.x0 + tx * kTile + px, i = c.y0 + ty * kTile + py;
         p.in = ihex < xlim && i < ylim;
         p.ihex = min(ihex, xlim - 1);
         p.i = min(i, ylim - 1);
@@ -1801,7 +1802,8 @@ __device__ __forceinline__ void image_tile(const DevSet& d, const Cover& c, doub
     const int t = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     if (t >= c.total) return;
     // (Gaussian cylinders, quadrature: every wave of the workgroup holds quadrant blockIdx.z)
-    const CoverPix p = cover_pixel(c, t, KIND == K_CYL_GAUSS_Q ? (int)blockIdx.z : (int)threadIdx.x >> 6);
+    const CoverPix p = cover_pixel(c, t, (int)blockIdx.x, (int)blockIdx.y,  // (the grid is tiles_x wide)
+                                   KIND == K_CYL_GAUSS_Q ? (int)blockIdx.z : (int)threadIdx.x >> 6);
     PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
     if (!__ballot(p.in)) return;
     const Radial* rv = nullptr;
@@ -1991,7 +1993,7 @@ __device__ __forceinline__ void fit_tile(const FitSet& f, int tile, double* __re
     __shared__ int s_cnt[kBlock / 64], s_nan[kBlock / 64];
     double term = 0.0;
     int nz = 0, isnan_ = 0;
-    const CoverPix p = cover_pixel(f.cov, tile, (int)threadIdx.x >> 6);
+    const CoverPix p = cover_pixel(f.cov, tile, tile % f.cov.tiles_x, tile / f.cov.tiles_x, (int)threadIdx.x >> 6);
     // All lanes of a wave with a pixel evaluate one (wave-wide |q| ranges need all 64 lanes);
     // lanes outside the fit array or masked discard the value.
     if (__ballot(p.in)) {
@@ -2094,7 +2096,7 @@ __device__ __forceinline__ void image_batch_tiles(const FitSet* __restrict__ set
     if (t >= ntiles) return;
     const int2 st = tiles[t];
     const FitSet& f = sets[st.x];
-    const CoverPix p = cover_pixel(f.cov, st.y, (int)threadIdx.x >> 6);
+    const CoverPix p = cover_pixel(f.cov, st.y, st.y % f.cov.tiles_x, st.y / f.cov.tiles_x, (int)threadIdx.x >> 6);
     if (!__ballot(p.in)) return;
     PixQ P3{p.ihex, p.i, 0.0, 0.0, 0.0, false};
     const Radial* rv = nullptr;
