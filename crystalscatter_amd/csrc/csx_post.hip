@@ -241,7 +241,13 @@ __device__ __forceinline__ void fft_levels(double* xr, double* xi, int m, int li
 // Lines of one workgroup at size s: 256 bytes of neighbouring complex elements, in at most 64 KB
 // of LDS.  One column a workgroup (16 bytes of each line of memory) took 131 us for 256 images of
 // 128^2, where the contiguous pass took 31; load, both passes and output together 225 -> 71 us.
-inline int fft_lines(int s) { return std::min(std::min(s, 16), 4096 / s); }
+// Where that leaves most of the chip idle (one or two images), fewer, down to 64-byte pieces: one
+// image of 256^2 takes 69 us, 87 with sixteen lines, 81 with one.
+inline int fft_lines(int s, int nimg) {
+    int lines = std::min(std::min(s, 16), 4096 / s);
+    while (lines > 4 && (int64_t)nimg * (s / lines) < 128) lines /= 2;
+    return lines;
+}
 
 // First pass, along the first index (stride s): c[y][x] = d[x + s y] / max, imaginary part 0,
 // transformed, to buf.
@@ -702,7 +708,7 @@ int csx_post_ifft(csx_ctx* c, const double* d_in, int s, int nimg, int forward, 
     hipStream_t st = (hipStream_t)csx_ctx_stream(c);
     PCHK(c, hipMemcpyAsync(d_tw, tw.data(), tw.size() * sizeof(double2), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_max0, dim3(nimg), dim3(kStat), 0, st, d_in, len, mx);
-    const int lines = fft_lines(s), threads = std::min(512, std::max(64, lines * s / 2));
+    const int lines = fft_lines(s, nimg), threads = std::min(512, std::max(64, lines * s / 2));
     const size_t shm = 2 * (size_t)lines * s * sizeof(double);
     hipLaunchKernelGGL(k_fft_first, dim3(s / lines, nimg), dim3(threads), shm, st, d_in, mx, buf, m, lines, d_tw,
                        forward);

@@ -195,6 +195,18 @@ def test_fft_sizes(oracle_lib, s, forward, out_type, swap):
         assert np.abs(got[k] - want).max() <= 1e-13 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("s,n", [(16, 128), (64, 32), (128, 16), (256, 8)])
+def test_fft_of_many_images_is_that_of_each(s, n):
+    """Sixteen lines a workgroup (many images) against four (one image): the same butterflies."""
+    import torch
+    from crystalscatter_amd import aidata
+    x = torch.from_numpy(np.random.default_rng(s).random((n, s * s)) + 0.1).cuda()
+    ctx = Context(0)
+    many = aidata.post_ifft(ctx, x, s, out_type=2, swap=True)
+    for k in (0, n // 2, n - 1):
+        assert torch.equal(many[k], aidata.post_ifft(ctx, x[k:k + 1].contiguous(), s, out_type=2, swap=True)[0])
+
+
 @pytest.mark.parametrize("name,lin", [("fcc_rphi", 0), ("sphere_lin", 1)])
 def test_scale_intensity_matches_the_reference(name, lin):
     import torch
