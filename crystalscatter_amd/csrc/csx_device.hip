@@ -1430,9 +1430,10 @@ __device__ __forceinline__ double pixel_no_lattice(const DevSet& d, double qx, d
 
 // Value v[0] of the pixel P3 (its exact q vector is computed here unless the caller has it) and,
 // with npx = 2, v[1] of its mirror image (-ihex, -i); npx = 0: a lane without a pixel, which
-// repeats one.  rv: its radial-table entry (midpoint grid, radial kinds) or null.  Only the lattice kinds in mixed precision take mirror images: in the
-// midpoint grid the peak sum at -q is the one at q (each Friedel pair swaps its two terms), and
-// so is every factor of |q|; the oriented cylinder's rod factor is evaluated at both.
+// repeats one.  rv: its radial-table entry (midpoint grid, radial kinds) or null.  Only the
+// lattice kinds in mixed precision take mirror images: in the midpoint grid the peak sum at -q is
+// the one at q (each Friedel pair swaps its two terms), and so is every factor of |q|; the
+// oriented cylinder's rod factor is evaluated at both.
 // MODE kHot: *cold reports a pixel that needs an FP64 path, with its state in *cp; kFix:
 // finishes such a pixel from *cp.
 template <int KIND, int PREC, int MODE = kFull>
@@ -3658,7 +3659,8 @@ int csx_fit_fqs_noalloc(csx_ctx* c, int w, int h, const csx_mask* mask, int prec
     f.w = w;
     f.h = h;
     const int kind = kind_of(s.combo_key);
-    f.cov = fit_cover(f, kind, precision);  // never more workgroups than the checked tiles
+    f.cov = fit_cover(f, kind, precision);
+    // (the tiles checked above or fewer, but for a single tile, whose mirror cover has two workgroups)
     if (f.cov.total > kScratchTiles) return fail(c, CSX_E_ARG, "csx_fit_fqs_noalloc: too many tiles");
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     DISPATCH_KIND(kind, precision, launch_fit_one, f, f.cov.total, d_fqs, part, c->stream);
@@ -4015,8 +4017,8 @@ int csx_fit_batch_run(csx_ctx* c, int precision, double* h_sums, int64_t* h_cnts
 // the device addresses of every set's tables filled in; one H2D copy on the context's stream
 // (or a node of the round's graph).  Returns the device addresses of the records, of the flat
 // tile list (written on the device by k_prep_sets) and of the tile counts.
-static int batch_upload(csx_ctx* c, int precision, int* n_groups, const FitSet** d_sets, const int2** d_tiles, const int** d_ntiles,
-                        size_t* bytes = nullptr) {
+static int batch_upload(csx_ctx* c, int precision, int* n_groups, const FitSet** d_sets, const int2** d_tiles,
+                        const int** d_ntiles, size_t* bytes = nullptr) {
     const int nsets = (int)c->bsets.size();
     // the sets' workgroups in the launch's precision
     int ntiles = 0;
@@ -4177,7 +4179,8 @@ int csx_fit_batch_launch(csx_ctx* c, int precision) {
     HIPCHK(c, c->bsums_d.ensure(nsets * sizeof(SetSum)));
     HIPCHK(c, c->bres.reserve(nsets * sizeof(SetSum)));
     const int kind = kind_of(c->bsets[0].d.s.combo_key);
-    const int variant = c->tune_force >= 0 ? c->tune_force : tune_variant(kind, tune_size_class(c->bntiles_total, nsets));
+    const int variant =
+        c->tune_force >= 0 ? c->tune_force : tune_variant(kind, tune_size_class(c->bntiles_total, nsets));
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     if (c->use_graph) {
         const void* fn = nullptr;

@@ -158,7 +158,8 @@ __device__ __forceinline__ void embed_rows(int r0, int n, int nsets, const float
 // acc[i][j] += the wave's 16 NI features x kPM rows of W . act^T over k < K (W in fragment order,
 // kH rows).
 template <int K, int NI, bool PREFETCH>
-__device__ __forceinline__ void layer_product(const bf16* __restrict__ W, const bf16* act, int wn, f32x4 (&acc)[NI][4]) {
+__device__ __forceinline__ void layer_product(const bf16* __restrict__ W, const bf16* act, int wn,
+                                              f32x4 (&acc)[NI][4]) {
     const int lane = threadIdx.x & 63, fr = lane & 15, fk = (lane >> 4) * 8;
     const bf16* wp = W + (size_t)(wn / 16) * 512 + lane * 8;
     if constexpr (PREFETCH) {

@@ -182,8 +182,8 @@ struct SphereTable {
 
 // Homogeneous sphere, Source/sc_calc_generic_cpu.cpp:2509-2543.  The inner sums are four orders
 // at a time: a sum in double of long double terms is a chain through memory, about as long as
-// six products, and one order waits for it 7381 times a set.  Same doubles as one by one.  A preparation of an FCC
-// set of spheres: 244 us one by one, 73 us like this (one thread).
+// six products, and one order waits for it 7381 times a set.  Same doubles as one by one.  A
+// preparation of an FCC set of spheres: 244 us one by one, 73 us like this (one thread).
 void coef_sphere(PreparedSet& P, double z, double xr2z, CoefState& cs) {
     static const SphereTable T;
     static_assert(kNN % 4 == 0, "orders are taken four at a time");
