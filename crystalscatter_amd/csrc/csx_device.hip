@@ -718,7 +718,7 @@ struct ColdPix {
     int ihex, i;
     double inten, dropped;
     int b0, b1, band0, band1;
-    int flags;  // 1: near-one pairs in the window, 4: placeholder lane, 8: its mirror image as well
+    int flags;  // 1: near-one pairs in the window, 8: its mirror image as well
     int pad;
 };
 
@@ -1527,7 +1527,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 // one queue slot holds the cold pixels of one hot wave: the same window
                 W = Window{uniform_i(cp->b0), uniform_i(cp->b1), uniform_i(cp->band0), uniform_i(cp->band1),
                            (cp->flags & 1) != 0};
-                if (W.near && !(cp->flags & 4)) {
+                if (W.near && npx > 0) {
                     PixelConsts L;
                     PixelConsts64 L64;
                     if constexpr (kPrecise) pixel_dirs64(s, P3, q, L64);
@@ -1566,8 +1566,9 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 }
                 return any;
             };
-            // placeholder lanes of the fix pass take no FP64 path
-            const bool live = MODE != kFix || !(cp->flags & 4);
+            // lanes without a pixel take no FP64 path (of a strip's wave 48, each of which would
+            // have its pixel summed again for itself)
+            const bool live = npx > 0;
             const bool want2 = live && !need_exact && loose(inten, kPrecise ? kRelErrPrecise : kRelErrFP32);
             if constexpr (MODE == kHot) {
                 *cold = W.near || want2;
@@ -1576,7 +1577,7 @@ __device__ __forceinline__ void pixel_values(const DevSet& d, PixQ& P3, double* 
                 inten2 = inten;
             } else {
                 // straight to the full sum where the dropped mass alone is too coarse
-                bool want3 = need_exact || (want2 && loose(inten, 1.0e-13));
+                bool want3 = (live && need_exact) || (want2 && loose(inten, 1.0e-13));
                 const bool window = want2 && !want3;
                 if (__ballot(window)) {
                     if (window) need_q(s, P3);
@@ -1890,7 +1891,6 @@ k_image_lat_fix(const DevSet d, const Cover c, double* __restrict__ out, unsigne
         const bool have = (m >> lane) & 1ull;
         ColdPix cp = cq.ent[(size_t)slot * 64 + (have ? lane : __builtin_ctzll(m))];
         const bool mir = have && (cp.flags & 8);
-        if (!have) cp.flags = 4;
         PixQ P3{cp.ihex, cp.i, 0.0, 0.0, 0.0, false};
         const Radial* rv = nullptr;
         if (rtab) {
