@@ -93,10 +93,10 @@ struct Features {
 // orientation writes four 2-byte values.  The bias is added to the finished products.
 // Bound: the vector unit -- per row 1024 SiLU values at about 60 cycles each per wave of 64
 // (exp2 and reciprocal at quarter rate) and 32 sincosf, against 422 matrix cycles.  2.1 M rows of
-// inference: 1.26 ms (2.75 ms with H . W^T, IEEE divisions and row-major weights).  1.10 ms with
+// inference: 1.25 ms (2.75 ms with H . W^T, IEEE divisions and row-major weights).  1.10 ms with
 // the bare reciprocal, hardware sines of the phase in turns and the bias as the accumulators'
 // initial value, but then activations flip bf16 roundings and y moves by 8e-4 in norm.
-// Training, 65,536 rows: 0.16 ms, its phases between barriers (4 waves at 2 per SIMD: 0.22 ms),
+// Training, 65,536 rows: 0.17-0.19 ms, its phases between barriers (4 waves at 2 per SIMD: 0.22 ms),
 // for the 11 launches and 0.38 ms of the layer-by-layer passes.
 constexpr int kPM = 64;        // rows per block
 constexpr int kInferWaves = 4, kTrainWaves = 8;
