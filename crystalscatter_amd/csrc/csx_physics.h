@@ -415,9 +415,9 @@ __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, do
     if (!fser || (!pser && same)) {
         if constexpr (FAST) {
             // The factor is even but its argument carries +1e-9, so the mirror image's is another
-            // value unless p is 0 (all of a pattern of cylinders along the beam).  It is evaluated
-            // on its own: where p is not far above 1e-9 (the line across the rods, where p is a
-            // rounding error unless an axis lies on it) a step from p's value loses every digit.
+            // value unless p is 0.  It is evaluated on its own (2 us of a 512^2 pattern's 57): where
+            // p is not far above 1e-9 (the line across the rods, where p is a rounding error unless
+            // an axis lies on it) a step from p's value loses every digit.
             rod[0] = rod_p_fast(d, p);
             if constexpr (NV > 1) {
                 rod[1] = rod[0];
