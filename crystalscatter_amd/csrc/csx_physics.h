@@ -383,11 +383,14 @@ __device__ inline double fq_cyl_zdir(const DevSet& d, double limql, double qxs, 
 }
 
 // rod_p from the set's constants, for the mixed path, at the projection p + 1e-9: the power by
-// exp and log, one division.  On the line p = 0 the power is exactly 1, as rod_p's.
+// exp and log.  Near p = 0 what is left of 1 - cos / power are a few units in the last place of 1, and
+// the result is the reference's only with its roundings: the power is formed above 1 (where it
+// has half the resolution) and divides the cosine.  Multiplied by the power's reciprocal, long
+// rods with sigma_L > 0.3 came out up to 67% off on that line.
 __device__ __forceinline__ double rod_p_fast(const DevSet& d, double p) {
     const double arg = (p + 0.000000001) * d.cyl_ll, a2 = arg * arg;
-    const double E = exp(-0.5 * d.cyl_zl1 * log(1.0 + 4 * a2));
-    return d.cyl_rc * (1 - cos(d.cyl_zl1 * atan(2.0 * arg)) * E) * (1 / a2);
+    const double E = exp(0.5 * d.cyl_zl1 * log(1.0 + 4 * a2));
+    return d.cyl_rc * (1 - cos(d.cyl_zl1 * atan(2.0 * arg)) / E) * (1 / a2);
 }
 
 // pq_cyl_long_zdir and fq_cyl_long at one pixel: the same values (FAST: to rounding), with the
@@ -416,8 +419,8 @@ __device__ inline void cyl_long_both(const DevSet& d, double q, double limql, do
         if constexpr (FAST) {
             // The factor is even but its argument carries +1e-9, so the mirror image's is another
             // value unless p is 0.  It is evaluated on its own (2 us of a 512^2 pattern's 57): where
-            // p is not far above 1e-9 (the line across the rods, where p is a rounding error unless
-            // an axis lies on it) a step from p's value loses every digit.
+            // p is not far above 1e-9 (the line across the rods, where p is a rounding error or 0)
+            // a step from p's value loses every digit.
             rod[0] = rod_p_fast(d, p);
             if constexpr (NV > 1) {
                 rod[1] = rod[0];
